@@ -1,29 +1,28 @@
-// GGUF-block matmuls on the f16 MFMA (Q4_K, Q6_K, Q4_0): the prefill GEMM g_gemm_{fmt}_{store|acc|swiglu}
-// (S/gen_gemm.py:535-703) and the MoE grouped expert GEMMs g_moe_ggu_{fmt}[_fused]_k{H} / g_moe_gdn_{fmt}_k{FE}
-// (S/gen_moe.py:1126-1228; the Q4_0 expert staging of S/moe_q4_0.py:11-61).
+// The GGUF-block matmuls on the f16 MFMA (Q4_K, Q6_K, Q4_0): the entry points' checks and dispatch, to the tile GEMM
+// (gemm_tile_kernel.hpp), the Q4_K store / acc GEMM of few rows (gemm_dense.hip) or the grouped GEMMs of few rows an
+// expert (grouped_q4k_narrow.hip); and the kernel below for gate/up pairs in two formats (QMM_GATE_UP):
+// g_gemm_{fg}_{fu}_swiglu and g_moe_ggu_{fg}_{fu} (S/gen_gemm.py:535-703, S/gen_moe.py:1126-1141).
 //
-//   dense   Y[r, c]   = (acc ? Y[r, c] : 0) + inv[r] sum_k X16[r, k] W[c, k]
+//   swiglu  Y[r, c]   = silu(inv[r] sum_k X16[r, k] Wg[c, k]) (inv[r] sum_k X16[r, k] Wu[c, k])
 //   gu      act[r, c] = act_fn(inv[t] sum_k X16[t, k] Wg[e][c, k] + bg[e, c], inv[t] sum_k X16[t, k] Wu[e][c, k]
 //                       + bu[e, c]),  t = rowmap[r] / KU  (rows gathered from the token rows)
-//   dn      ys[r, c]  = inv[r] sum_k A16[r, k] Wd[e][c, k] + bd[e, c]            (rows already sorted)
 //
 // for every row r of every 64-row tile whose expert e = tile_info[tile, 0] >= 0; rows with rowmap[r] < 0 are not
-// written. The optional expert biases (gpt-oss ffn_{gate,up,down}_exps.bias) are added after the row
-// inverse, before the activation (_gemm_bias_act, S/gen_moe.py:958-1007). X16 / A16 are the row-scaled f16 operands the reference's g_row_scale_f16[_tiles] produces
-// (S/gen_llm.py:1843-1915, S/gen_moe.py:503-527) and inv = their scales[row, 1]. W is dequantized to f16 in
-// registers the way the reference stages it: Q4_K w = fma_f16(f16(q), f16(d sc), f16(-dmin m)) (S/gen_gemm.py:499-530),
-// Q6_K w = fma_f16(f16(q), f16(d sc), f16(-32 d sc)) (S/gen_gemm.py:369-444), Q4_0 w = f16(q - 8) * d with one f16
-// rounding (S/moe_q4_0.py:11-38: exactly f16(d (q - 8)) for every finite f16 d). fp32 accumulation throughout.
+// written. The optional expert biases (gpt-oss ffn_{gate,up}_exps.bias) are added after the row inverse, before the
+// activation (_gemm_bias_act, S/gen_moe.py:958-1007). X16 is the row-scaled f16 operand of g_row_scale_f16[_tiles]
+// (S/gen_llm.py:1843-1915, S/gen_moe.py:503-527) and inv = its scales[row, 1]. W is dequantized to f16 in registers the
+// way the reference stages it: Q4_K w = fma_f16(f16(q), f16(d sc), f16(-dmin m)) (S/gen_gemm.py:499-530), Q6_K
+// w = fma_f16(f16(q), f16(d sc), f16(-32 d sc)) (S/gen_gemm.py:369-444), Q4_0 w = f16(q - 8) * d with one f16 rounding
+// (S/moe_q4_0.py:11-38). fp32 accumulation throughout.
 //
-// Tiling (gfx950, wave64). A workgroup has four waves and one 64-row tile. Dense and dn: the tile is 64 x 128 and
-// wave (nh, kh) computes the 64 x 64 quadrant nh over K-half kh; gu: the tile is 64 x 64 and wave (mat, kh)
-// computes it for matrix mat (gate, up) over K-half kh. Each wave holds 2 x 2 v_mfma_f32_32x32x16_f16
-// accumulators. The K-halves are summed through LDS at the end in a fixed order (and, for gu, the up result is
-// handed to the gate wave for the activation). A step is one 64-value page of a super-block: the activation rows
-// of both K-halves (2 x 64 x 64 f16) are staged in LDS, double-buffered, one barrier per step; each wave streams
-// its own 64 weight columns straight into registers and dequantizes them there, so weights never touch LDS. Loads
-// run DEPTH steps ahead of the math through register rings; the loads are unconditional (clamped addresses), so no
-// branch splits the load stream and the compiler keeps them in flight.
+// Tiling (gfx950, wave64). A workgroup has four waves and one 64 x 64 tile; wave (mat, kh) computes it for matrix mat
+// (gate, up) over K-half kh, in 2 x 2 v_mfma_f32_32x32x16_f16 accumulators, the up waves in the up matrix's format. The
+// K-halves are summed through LDS at the end in a fixed order, and the up result is handed to the gate wave for the
+// activation. A step is one 64-value page of a super-block: the activation rows of both K-halves (2 x 64 x 64 f16) are
+// staged in LDS, double-buffered, one barrier per step; each wave streams its own 64 weight columns straight into
+// registers and dequantizes them there, so weights never touch LDS. Loads run DEPTH steps ahead of the math through
+// register rings; the loads are unconditional (clamped addresses), so no branch splits the load stream and the compiler
+// keeps them in flight.
 //
 // MFMA operand order. Lane l of a 32x32x16 step holds 8 K values of row/column l % 32, octet l / 32. Q4_K / Q6_K:
 // lane half h takes code bytes 16h .. 16h+15 of a page, i.e. values 16h .. 16h+15 of both of the page's sub-blocks
@@ -32,12 +31,13 @@
 // the block's values 0..15 and high nibbles (gl = 1) values 16..31: step position 32 h + 16 gl + 8 s2. The A fragment
 // is read from LDS at the same K.
 //
-// Tile order is XCD-aware: consecutive tile ids land on one XCD (dense: the M tiles of one N tile, which share
+// Tile order is XCD-aware: consecutive tile ids land on one XCD (swiglu: the M tiles of one N tile, which share
 // weight columns; grouped: the column blocks of one expert tile, which share its activation rows).
 #include <type_traits>
 
 #include "common.hpp"
 #include "deq_f16.hpp"
+#include "gemm_tile.hpp"
 
 using namespace qmm;
 
@@ -51,56 +51,39 @@ constexpr int kDepth = QMM_GEMM_DEPTH;   // steps of loads in flight per wave (e
 static_assert(kDepth % 2 == 0, "the LDS double buffer follows the step parity");
 constexpr int APITCH = KSTEP + 8;   // f16 per LDS row: 144 bytes, rows 16-byte aligned, reads 2-way at most
 
-// kDense: Y (+)= X W^T; kSwiglu: Y = silu(X Wg^T inv) (X Wu^T inv) over dense rows (the GEMM's swiglu mode);
-// kGU / kDN: the grouped gate/up and down GEMMs over bucketed expert tiles
-enum Kind { kDense = 0, kGU = 1, kDN = 2, kSwiglu = 3 };
+// kSwiglu: Y = silu(X Wg^T inv) (X Wu^T inv) over dense rows (the GEMM's swiglu mode); kGU: the grouped gate/up GEMM over
+// bucketed expert tiles
+enum Kind { kGU = 1, kSwiglu = 3 };
 // weight formats: GGUF Q4_K (144-byte super-blocks), Q6_K (210), Q4_0 (18-byte blocks of 32)
 enum WFmt { kWQ4K = 0, kWQ6K = 1, kWQ40 = 2 };
 
 struct Args {
-  int M, N, K;                 // dense: rows; grouped: rows of the sorted output (max_tiles * 64)
-  const _Float16 *x16;         // activation rows (dense / dn: [M, K]; gu: token rows [x_rows, K])
+  int M, N, K;                 // swiglu: rows; grouped: rows of the sorted output (max_tiles * 64)
+  const _Float16 *x16;         // activation rows (gu: token rows) [x_rows, K]
   const float *scales;         // [rows of x16, 2] or NULL
-  int x_rows;                  // rows of x16 (gu)
-  const u8 *w, *w2;            // dense: W; grouped: expert tensors (gu: gate, up; fused: w only)
-  int64_t ebytes;              // bytes of one expert's matrix (grouped)
-  int64_t ebytes2;             // gu, two tensors: bytes of one expert's up matrix (its own format's rows)
-  int64_t up_off;              // gu: byte offset of the up matrix from the gate matrix of an expert (fused)
+  int x_rows;                  // rows of x16
+  const u8 *w, *w2;            // gate, up (grouped: expert tensors)
+  int64_t ebytes, ebytes2;     // grouped: bytes of one expert's gate / up matrix
   const int32_t *tile_info, *rowmap;
-  const float *bias, *bias2;   // grouped: per-expert output biases [E, N] (gu: gate, up; dn: bias only) or NULL
+  const float *bias, *bias2;   // grouped: per-expert output biases [E, N] (gate, up) or NULL
   int KU, E, act;
   void *y;
   int tiles_m, n_blocks, tiles_total;
 };
 
-// Scale tables: a workgroup decodes the (d sc, -dmin m) f16 pair of every sub-block of its 128 weight columns once
-// into LDS (4 bytes per sub-block, 16 (K + 64) bytes) when that fits (K <= kStagedMaxK); each step then reads its two
-// pairs per column with one 8-byte LDS read instead of loading and decoding the super-block header again.
-constexpr int kStagedMaxK = 6144;
-
-// WF2: the up matrix's format when it differs from the gate's (kGU / kSwiglu of a QMM_GATE_UP pair): the up waves
-// load and dequantize in their own format, with their own row stride, the gate waves in WF.
-// TL: Q4_K weights in the tiled layout QMM_Q4_KT (K % 512 == 0, N % 16 == 0): the lane reads the same code bytes and
-// headers at their tiled addresses (column c's 16-row block at (c / 16) 16 RB; super-block sb of its row r = c % 16
-// is half sb % 2 of unit sb / 2 of 4608 bytes: header at 16 (2 r + sb % 2), page p's bytes 16 h .. + 15 in plane
-// 2 (p % 2) + h at 512 + 1024 (2 (p % 2) + h) + 16 (4 r + 2 (sb % 2) + p / 2)), so the results are the GGUF call's.
-template <int KIND, bool ACC, bool BF16OUT, int DEPTH, bool STAGED, int WF, int KS, int WF2 = WF, bool TL = false>
-__global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
+// WF / WF2: the gate and the up matrix's formats; the gate waves load and dequantize in WF, the up waves in WF2 with
+// their own row stride.
+template <int KIND, bool BF16OUT, int DEPTH, int WF, int KS, int WF2>
+__global__ __launch_bounds__(128 * KS, 1) void pair_mfma_kernel(Args a) {
   constexpr int NT = 128 * KS;   // threads: 2 column halves (or matrices) x KS K-parts
-  constexpr bool MIXED = WF2 != WF;
-  static_assert(!(WF != kWQ4K && STAGED), "Q6_K / Q4_0 scales are read with the codes");
-  constexpr bool kTwoW = KIND == kGU || KIND == kSwiglu;        // two weight matrices (gate, up): wave pairs
-  static_assert(!MIXED || (kTwoW && !STAGED), "a second format is the up matrix's of gate/up, scales read with codes");
-  static_assert(!TL || (WF == kWQ4K && !MIXED), "the tiled layout holds Q4_K");
-  constexpr bool kDenseRows = KIND == kDense || KIND == kSwiglu;  // rows m0 .. m0 + 63 of x, tiles row-major
-  constexpr int BN = kTwoW ? 64 : 128;
-  extern __shared__ __align__(16) u32 scl[];   // STAGED: [128 columns][K / 32 + 2] (dsc | nmn << 16)
+  constexpr bool kDenseRows = KIND == kSwiglu;  // rows m0 .. m0 + 63 of x, tiles row-major
+  constexpr int BN = 64;
   __shared__ __align__(16) _Float16 As[2][KS][BM][APITCH];   // [buffer][K-part][row][k]
   __shared__ int src_row[BM];
   __shared__ float rinv[BM];   // the row's inverse activation scale (1 without scales)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int sel = wave & 1, kh = wave >> 1;   // sel: N-half (dense, dn) or matrix (gu: 0 gate, 1 up); kh: K-part
-  const bool upw = MIXED && sel == 1;         // a wave of the up matrix in its own format
+  const int sel = wave & 1, kh = wave >> 1;   // sel: matrix (0 gate, 1 up); kh: K-part
+  const bool upw = sel == 1;                  // a wave of the up matrix in its own format
   const int M = a.M, N = a.N, K = a.K;
 
   int m0, n0, expert = 0;
@@ -128,12 +111,10 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
   if (tid < BM) {
     int src;
     if constexpr (kDenseRows) src = m0 + tid < M ? m0 + tid : -1;
-    else if constexpr (KIND == kGU) {
+    else {
       const int rm = a.rowmap[m0 + tid];
       src = rm >= 0 ? rm / a.KU : -1;
       src = src < a.x_rows ? src : -1;
-    } else {
-      src = a.rowmap[m0 + tid] >= 0 ? m0 + tid : -1;
     }
     src_row[tid] = src;
     rinv[tid] = (a.scales && src >= 0) ? a.scales[2 * src + 1] : 1.f;
@@ -181,31 +162,17 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
 
   // ---- B: this lane's two weight columns and code half
   const int h = lane >> 5, lc = lane & 31;
-  const u8 *wbase;
-  if constexpr (KIND == kDense) wbase = a.w;
-  else if constexpr (KIND == kSwiglu) wbase = sel ? a.w2 : a.w;
-  else if constexpr (KIND == kGU) {
-    const u8 *g = a.w + (int64_t)expert * a.ebytes;
-    wbase = sel ? (a.w2 ? a.w2 + (int64_t)expert * a.ebytes2 : g + a.up_off) : g;
-  } else {
-    wbase = a.w + (int64_t)expert * a.ebytes;
-  }
-  const u8 *wcol[2];   // GGUF: the column's row; tiled: its 16-row block
-  int tco[2], tho[2];  // tiled: the column's code and header offsets in a unit
+  const u8 *wbase = sel ? a.w2 : a.w;
+  if constexpr (KIND == kGU) wbase += (int64_t)expert * (sel ? a.ebytes2 : a.ebytes);
+  const u8 *wcol[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    int c = n0 + (kTwoW ? 0 : sel * 64) + 32 * j + lc;
+    int c = n0 + 32 * j + lc;
     c = c < N ? c : N - 1;
-    wcol[j] = TL ? wbase + (int64_t)(c >> 4) * 16 * RB : wbase + (int64_t)c * RB;
-    tco[j] = 512 + 1024 * h + 64 * (c & 15);
-    tho[j] = 32 * (c & 15);
+    wcol[j] = wbase + (int64_t)c * RB;
   }
   auto b_code = [&](int j, int s) -> uint4 {
     const int gs = kh * S0 + (s < S0 ? s : S0 - 1);
-    if constexpr (TL) {
-      const int sb = gs >> 2, p = gs & 3;
-      return ld16(wcol[j] + tco[j] + (int64_t)(sb >> 1) * 4608 + 2048 * (p & 1) + 32 * (sb & 1) + 16 * (p >> 1));
-    }
     return ld16(wcol[j] + (int64_t)(gs >> 2) * 144 + 16 + 32 * (gs & 3) + 16 * h);
   };
   // Q6_K page gs & 3 = (half, jh): groups j = 2 jh (ql bytes 64 half + l) and 2 jh + 1 (64 half + 32 + l), both with
@@ -229,54 +196,8 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
   };
   auto b_head = [&](int j, int s) -> uint4 {
     const int sb = (kh * S0 + (s < S0 ? s : S0 - 1)) >> 2;
-    if constexpr (TL) return ld16(wcol[j] + tho[j] + (int64_t)(sb >> 1) * 4608 + 16 * (sb & 1));
     return ld16(wcol[j] + (int64_t)sb * 144);
   };
-  // sub-blocks per column, and the staged table's row pitch in dwords: two more than K / 32 (a multiple of 8), so
-  // the 32 columns a wave reads at once start two banks apart instead of all in one bank
-  const int SB = K / 32, SBP = SB + 2;
-  if constexpr (STAGED) {
-    // local column cl = sel * 64 + 32 j + lc: dense / dn columns n0 + cl, gu: gate n0 + cl (cl < 64), up n0 + cl - 64
-    // every header of the workgroup's columns, kHdrBatch loads in flight per thread before any is decoded
-    constexpr int kHdrBatch = 4;
-    const int nh = 128 * (K / 256);
-    for (int b0 = 0; b0 < nh; b0 += kHdrBatch * NT) {
-      uint4 hd[kHdrBatch];
-#pragma unroll
-      for (int q = 0; q < kHdrBatch; ++q) {
-        int i = b0 + tid + NT * q;
-        i = i < nh ? i : nh - 1;
-        const int cl = i / (K / 256), b = i % (K / 256);
-        const int msel = cl >> 6;
-        const u8 *mb;
-        if constexpr (KIND == kDense) mb = a.w;
-        else if constexpr (KIND == kSwiglu) mb = msel ? a.w2 : a.w;
-        else if constexpr (KIND == kGU) {
-          const u8 *g = a.w + (int64_t)expert * a.ebytes;
-          mb = msel ? (a.w2 ? a.w2 + (int64_t)expert * a.ebytes2 : g + a.up_off) : g;
-        } else {
-          mb = a.w + (int64_t)expert * a.ebytes;
-        }
-        int c = n0 + (kTwoW ? cl - 64 * msel : cl);
-        c = c < N ? c : N - 1;
-        hd[q] = TL ? ld16(mb + (int64_t)(c >> 4) * 16 * RB + 32 * (c & 15) + (int64_t)(b >> 1) * 4608 + 16 * (b & 1))
-                   : ld16(mb + (int64_t)c * RB + (int64_t)b * 144);
-      }
-#pragma unroll
-      for (int q = 0; q < kHdrBatch; ++q) {
-        const int i = b0 + tid + NT * q;
-        if (i >= nh) continue;
-        const int cl = i / (K / 256), b = i % (K / 256);
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-          h2 dsc, nmn;
-          sub_scale(hd[q], g, dsc, nmn);
-          scl[cl * SBP + 8 * b + g] = (u32)__builtin_bit_cast(u16, dsc[0]) | ((u32)__builtin_bit_cast(u16, nmn[0]) << 16);
-        }
-      }
-    }
-  }
-
   f32x16 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -304,13 +225,12 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
         b_q40(j, st, cring[slot][j], q6d[slot][j]);
       } else {
         cring[slot][j] = b_code(j, st);
-        if constexpr (!STAGED) hring[slot][j] = b_head(j, st);
+        hring[slot][j] = b_head(j, st);
       }
     }
   };
   auto load_b = [&](int slot, int st) __attribute__((always_inline)) {
-    if constexpr (!MIXED) load_b_f(std::integral_constant<int, WF>{}, slot, st);
-    else if (upw) load_b_f(std::integral_constant<int, WF2>{}, slot, st);
+    if (upw) load_b_f(std::integral_constant<int, WF2>{}, slot, st);
     else load_b_f(std::integral_constant<int, WF>{}, slot, st);
   };
   // The prologue issues its loads in the loop's own order (a step issues the weights of step s + DEPTH, then the
@@ -341,12 +261,6 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
       const int buf = u & 1;   // DEPTH is even, so s & 1 == u & 1
       const int gstep = kh * S0 + (s < S0 ? s : S0 - 1);
       const int page = gstep & 3;
-      typedef __attribute__((ext_vector_type(2))) u32 u32x2;
-      u32x2 sp[2];
-      if constexpr (STAGED) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) sp[j] = *reinterpret_cast<const u32x2 *>(&scl[(sel * 64 + 32 * j + lc) * SBP + 2 * gstep]);
-      }
       auto math = [&](auto fc) __attribute__((always_inline)) {
         constexpr int F = decltype(fc)::value;
   #pragma unroll
@@ -364,10 +278,6 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
               const _Float16 a16 = (_Float16)sv, b16 = (_Float16)(-32.f * sv);
               dsc[j] = h2{a16, a16};
               nmn[j] = h2{b16, b16};
-            } else if constexpr (STAGED) {
-              const u32 v = gl ? sp[j].y : sp[j].x;
-              dsc[j] = as_h2((v & 0xFFFFu) * 0x10001u);
-              nmn[j] = as_h2((v >> 16) * 0x10001u);
             } else {
               sub_scale(hring[u][j], 2 * page + gl, dsc[j], nmn[j]);
             }
@@ -408,8 +318,7 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
           }
         }
       };
-      if constexpr (!MIXED) math(std::integral_constant<int, WF>{});
-      else if (upw) math(std::integral_constant<int, WF2>{});
+      if (upw) math(std::integral_constant<int, WF2>{});
       else math(std::integral_constant<int, WF>{});
       load_b(u, s + DEPTH);
       const int nx = (u + 1) % DEPTH;
@@ -420,7 +329,7 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
     }
   }
 
-  // ---- sum the K-parts through LDS in a fixed tree: with four parts, 2 and 3 hand theirs to 0 and 1, then 1 to 0
+  // ---- sum the K-parts through LDS: part 1 hands its to part 0
   float *red = reinterpret_cast<float *>(&As[0][0][0][0]);   // [slot][sel][64 values][64 lanes]
   static_assert(sizeof(As) >= (KS / 2) * 2 * 64 * 64 * 4, "K-part reduction staging");
   auto red_at = [&](int sl, int i, int j, int r) -> float & {
@@ -446,23 +355,20 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
     }
     __syncthreads();
   };
-  if constexpr (KS == 4) hand(2, 2);
   hand(1, 1);
 
-  if constexpr (kTwoW) {
-    // the up wave (K-half 0) hands its result to the gate wave; every wave takes part in the barriers
-    __syncthreads();
-    if (kh == 0 && sel == 1) {
+  // the up wave (K-half 0) hands its result to the gate wave; every wave takes part in the barriers
+  __syncthreads();
+  if (kh == 0 && sel == 1) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) red_at(0, i, j, r) = acc[i][j][r];
-    }
-    __syncthreads();
-    if (sel == 1) return;
+        for (int r = 0; r < 16; ++r) red_at(0, i, j, r) = acc[i][j][r];
   }
+  __syncthreads();
+  if (sel == 1) return;
   if (kh != 0) return;
 
   // ---- epilogue
@@ -476,76 +382,23 @@ __global__ __launch_bounds__(128 * KS, 1) void q4k_mfma_kernel(Args a) {
       for (int r = 0; r < 16; ++r) {
         const int lr = 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
         const int row = m0 + lr;
-        const int col = n0 + (kTwoW ? 0 : sel * 64) + 32 * j + lc;
+        const int col = n0 + 32 * j + lc;
         if (col >= N || (kDenseRows && row >= M)) continue;
         const int src = src_row[lr];
         const int64_t o = (int64_t)row * N + col;
         if constexpr (kDenseRows) {
-          float v;
-          if constexpr (KIND == kSwiglu) v = act_fn(QMM_ACT_SILU, acc[i][j][r] * rinv[lr], red_at(0, i, j, r) * rinv[lr]);
-          else v = acc[i][j][r] * rinv[lr];
-          if constexpr (BF16OUT) {
-            if constexpr (ACC) v += bf16_to_f32(yb[o]);
-            yb[o] = (u16)f32_to_bf16_rne(v);
-          } else {
-            if constexpr (ACC) v += yf[o];
-            yf[o] = v;
-          }
+          const float v = act_fn(QMM_ACT_SILU, acc[i][j][r] * rinv[lr], red_at(0, i, j, r) * rinv[lr]);
+          if constexpr (BF16OUT) yb[o] = (u16)f32_to_bf16_rne(v);
+          else yf[o] = v;
         } else {
           if (src < 0) continue;   // a row without an assignment is not written
           const float inv = rinv[lr];
           const int64_t bo = (int64_t)expert * N + col;
           const float b = a.bias ? a.bias[bo] : 0.f;
-          float v;
-          if constexpr (KIND == kGU) {
-            const float b2 = a.bias2 ? a.bias2[bo] : 0.f;
-            v = act_fn(a.act, acc[i][j][r] * inv + b, red_at(0, i, j, r) * inv + b2);
-          } else {
-            v = acc[i][j][r] * inv + b;
-          }
-          yf[o] = v;
+          const float b2 = a.bias2 ? a.bias2[bo] : 0.f;
+          yf[o] = act_fn(a.act, acc[i][j][r] * inv + b, red_at(0, i, j, r) * inv + b2);
         }
       }
-}
-
-// Dense Q4_K rows (the prefill GEMM) run eight waves a workgroup, K in four parts: a 64 x 128 tile's workgroup then
-// has two waves a SIMD, so one wave's dequantization overlaps the other's MFMAs (the grid of a 512-row GEMM is one
-// workgroup a CU). The grouped GEMMs keep two K-parts (their expert tiles are many and their K short), and so does
-// Q6_K.
-template <int KIND, bool ACC, bool BF16OUT, int WF = kWQ4K, bool TL = false>
-int launch(const Args &a, hipStream_t s) {
-  constexpr bool kDenseRows = KIND == kDense || KIND == kSwiglu;
-  constexpr int KS = kDenseRows && WF != kWQ6K ? 4 : 2;   // Q6_K's wider rings would spill at two waves a SIMD
-  // staged scale tables beside the K-parts' activation buffers: 16 (K + 64) bytes, within 160 KB of LDS
-  constexpr int kMaxK = KS == 4 ? 5120 : kStagedMaxK;
-  const dim3 grid((unsigned)(kDenseRows ? 8 * ((a.tiles_total + 7) / 8) : 8 * a.n_blocks * ((a.tiles_m + 7) / 8)));
-  if constexpr (WF != kWQ4K) {
-    q4k_mfma_kernel<KIND, ACC, BF16OUT, kDepth, false, WF, KS><<<grid, 128 * KS, 0, s>>>(a);
-    return launch_status();
-  }
-  if (a.K <= kMaxK) {
-    const size_t dyn = (size_t)128 * (a.K / 32 + 2) * 4;
-    if (dyn > 32768) {   // beyond the default dynamic LDS limit: raised to the largest table this kernel stages
-      static std::atomic<unsigned> raised{0};
-      if (int st = raise_dyn_lds(
-              reinterpret_cast<const void *>(&q4k_mfma_kernel<KIND, ACC, BF16OUT, kDepth, true, kWQ4K, KS, kWQ4K, TL>),
-              (int)((size_t)128 * (kMaxK / 32 + 2) * 4), raised))
-        return st;
-    }
-    q4k_mfma_kernel<KIND, ACC, BF16OUT, kDepth, true, kWQ4K, KS, kWQ4K, TL><<<grid, 128 * KS, dyn, s>>>(a);
-  } else {
-    q4k_mfma_kernel<KIND, ACC, BF16OUT, kDepth, false, kWQ4K, KS, kWQ4K, TL><<<grid, 128 * KS, 0, s>>>(a);
-  }
-  return launch_status();
-}
-
-// the instantiation of (KIND, ACC, BF16OUT) for the weight format
-template <int KIND, bool ACC, bool BF16OUT>
-int launch_fmt(int fmt, const Args &a, hipStream_t s) {
-  if (fmt == QMM_Q6_K) return launch<KIND, ACC, BF16OUT, kWQ6K>(a, s);
-  if (fmt == QMM_Q4_0) return launch<KIND, ACC, BF16OUT, kWQ40>(a, s);
-  if (fmt == QMM_Q4_KT) return launch<KIND, ACC, BF16OUT, kWQ4K, true>(a, s);
-  return launch<KIND, ACC, BF16OUT, kWQ4K>(a, s);
 }
 
 // A gate/up pair in two formats (kSwiglu dense rows, kGU expert tiles): gate format WG, up format WU. Two K-parts
@@ -555,15 +408,14 @@ int launch_pair(const Args &a, hipStream_t s) {
   constexpr bool kDenseRows = KIND == kSwiglu;
   constexpr int KS = 2;
   const dim3 grid((unsigned)(kDenseRows ? 8 * ((a.tiles_total + 7) / 8) : 8 * a.n_blocks * ((a.tiles_m + 7) / 8)));
-  q4k_mfma_kernel<KIND, false, BF16OUT, kDepth, false, WG, KS, WU><<<grid, 128 * KS, 0, s>>>(a);
+  pair_mfma_kernel<KIND, BF16OUT, kDepth, WG, KS, WU><<<grid, 128 * KS, 0, s>>>(a);
   return launch_status();
 }
 int wfmt_of(int fmt) { return fmt == QMM_Q6_K ? kWQ6K : fmt == QMM_Q4_0 ? kWQ40 : kWQ4K; }
 template <int KIND, bool BF16OUT, int WG>
-int launch_pair_up(int wu, const Args &a, hipStream_t s) {
-  if (wu == kWQ6K) return launch_pair<KIND, BF16OUT, WG, kWQ6K>(a, s);
-  if (wu == kWQ40) return launch_pair<KIND, BF16OUT, WG, kWQ40>(a, s);
-  return launch_pair<KIND, BF16OUT, WG, kWQ4K>(a, s);
+int launch_pair_up(int wu, const Args &a, hipStream_t s) {   // two different formats (fmt_mixed)
+  constexpr int kA = WG == kWQ4K ? kWQ6K : kWQ4K, kB = WG == kWQ40 ? kWQ6K : kWQ40;
+  return wu == kA ? launch_pair<KIND, BF16OUT, WG, kA>(a, s) : launch_pair<KIND, BF16OUT, WG, kB>(a, s);
 }
 template <int KIND, bool BF16OUT>
 int launch_mixed(int fg, int fu, const Args &a, hipStream_t s) {
@@ -578,6 +430,36 @@ bool gguf_gemm_fmt(int f) { return f == QMM_Q4_K || f == QMM_Q6_K || f == QMM_Q4
 // even addresses; Q4_0: 2, 16-byte code runs read from even addresses)
 int64_t fmt_row_bytes(int fmt, int64_t k) {
   return fmt == QMM_Q4_0 ? k / 32 * 18 : k / 256 * (fmt == QMM_Q6_K ? 210 : 144);
+}
+int tile_gemm(int fmt, int kind, int shape, const TileArgs &a, hipStream_t s) {
+  if (fmt == QMM_Q6_K) return tile_gemm_q6k(kind, shape, a, s);
+  if (fmt == QMM_Q4_0) return tile_gemm_q40(kind, shape, a, s);
+  if (fmt == QMM_Q4_KT) return tile_gemm_q4kt(kind, shape, a, s);
+  return tile_gemm_q4k(kind, shape, a, s);
+}
+
+// The workgroup shape of a dense GEMM: the least ceil(tiles / 256 CUs) x (time of a CU's tile). Times in units of us at
+// K = 4096 (Q4_K; the ratios hold for the other formats and K within some 10 %), measured with a full chip: a 128 x 256
+// tile 64 (two workgroups a CU) or, K in two parts, 70 (58 where one round does), a 64 x 256 tile 41 (46), a 64 x 128
+// tile with K in four parts 30; the Q4_K store / acc kernel of gemm_dense.hip 26. So 2048 x 4096 outputs take the
+// two-part 128-row tiles (K = 12288: 194 us; 210 one part, 239 and 296 on 64 rows, 270 gemm_dense.hip), 2048 x 12288
+// one part (204; 222, 243, 359, 339), 333 x 12288 gate / up the 64 x 256 tiles (109; 113, 121, 140).
+constexpr int kDenseKernel = -1;
+int tile_shape(bool two, bool q4k, int64_t m, int64_t n) {
+  const int64_t cols = two ? 2 * n : n, m64 = (m + 63) / 64, m128 = (m + 127) / 128;
+  const int64_t n128 = (cols + 127) / 128, n256 = (cols + 255) / 256;
+  auto rounds = [](int64_t tiles) { return (tiles + 255) / 256; };
+  const int64_t r0 = rounds(m128 * n256), r2 = rounds(m64 * n256), r3 = rounds(m64 * n128);
+  int best = kT128x4x1;
+  int64_t cost = 64 * r0;
+  auto offer = [&](int shape, int64_t c) {
+    if (c < cost) { best = shape; cost = c; }
+  };
+  offer(kT128x4x2, r0 == 1 ? 58 : 70 * r0);
+  offer(kT64x4x1, r2 == 1 ? 46 : 41 * r2);
+  offer(kT64x2x4, 30 * r3);
+  if (q4k && !two) offer(kDenseKernel, 26 * r3);
+  return best;
 }
 int fmt_align(int fmt) { return fmt == QMM_Q4_K || fmt == QMM_Q4_KT ? 16 : fmt == QMM_Q6_K ? 4 : 2; }
 
@@ -610,24 +492,25 @@ extern "C" int qmm_gemm(int fmt, int mode, int64_t rows, int64_t k, int64_t n, c
   if (rows * k * 2 >= (1ll << 31)) return QMM_ERR_SHAPE;   // activation rows are addressed by a 32-bit buffer offset
   if (n * fmt_row_bytes(fmt, k) >= (1ll << 31) || n * fmt_row_bytes(fu, k) >= (1ll << 31))
     return QMM_ERR_SHAPE;   // so are the weight rows (buffer size, offsets)
-  Args a{};
-  a.M = (int)rows; a.N = (int)n; a.K = (int)k;
-  a.x16 = static_cast<const _Float16 *>(x); a.scales = scales; a.x_rows = (int)rows;
-  a.w = static_cast<const u8 *>(w); a.w2 = static_cast<const u8 *>(w2); a.y = y;
-  a.tiles_m = (int)((rows + BM - 1) / BM);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool acc = mode == QMM_GEMM_ACC, bf = y_dtype == QMM_BF16;
-  if (mode == QMM_GEMM_SWIGLU) {   // 64 output columns a workgroup: its wave pairs take the gate and the up matrix
-    a.tiles_total = a.tiles_m * (int)((n + 63) / 64);
-    if (mixed) return bf ? launch_mixed<kSwiglu, true>(fmt, fu, a, s) : launch_mixed<kSwiglu, false>(fmt, fu, a, s);
-    return bf ? launch_fmt<kSwiglu, false, true>(fmt, a, s) : launch_fmt<kSwiglu, false, false>(fmt, a, s);
+  if (mixed) {
+    Args a{};
+    a.M = (int)rows; a.N = (int)n; a.K = (int)k;
+    a.x16 = static_cast<const _Float16 *>(x); a.scales = scales; a.x_rows = (int)rows;
+    a.w = static_cast<const u8 *>(w); a.w2 = static_cast<const u8 *>(w2); a.y = y;
+    a.tiles_m = (int)((rows + BM - 1) / BM);
+    a.tiles_total = a.tiles_m * (int)((n + 63) / 64);   // 64 output columns a workgroup: wave pairs take gate and up
+    return bf ? launch_mixed<kSwiglu, true>(fmt, fu, a, s) : launch_mixed<kSwiglu, false>(fmt, fu, a, s);
   }
-  if (fmt == QMM_Q4_K || tiled) return qmm_gemm_q4k_dense(acc, tiled, rows, k, n, x, scales, w, y, bf, s);
-  a.tiles_total = a.tiles_m * (int)((n + 127) / 128);
-  if (acc && bf) return launch_fmt<kDense, true, true>(fmt, a, s);
-  if (acc) return launch_fmt<kDense, true, false>(fmt, a, s);
-  if (bf) return launch_fmt<kDense, false, true>(fmt, a, s);
-  return launch_fmt<kDense, false, false>(fmt, a, s);
+  const int shape = tile_shape(mode == QMM_GEMM_SWIGLU, fmt == QMM_Q4_K || tiled, rows, n);
+  if (shape == kDenseKernel) return qmm_gemm_q4k_dense(acc, tiled, rows, k, n, x, scales, w, y, bf, s);
+  TileArgs t{};
+  t.M = (int)rows; t.N = (int)n; t.K = (int)k;
+  t.x16 = static_cast<const _Float16 *>(x); t.scales = scales; t.x_rows = (int)rows;
+  t.w = static_cast<const u8 *>(w); t.w2 = static_cast<const u8 *>(w2); t.y = y;
+  t.acc = acc; t.y_bf16 = bf;
+  return tile_gemm(fmt, mode == QMM_GEMM_SWIGLU ? kTSwiglu : kTDense, shape, t, s);
 }
 
 int qmm_grouped_q4k_narrow(int tiled, int mode, int fused, int act, int64_t max_tiles, int64_t k, int64_t n, int E,
@@ -661,7 +544,6 @@ int qmm_grouped_q4k(int fmt, int mode, int fused, int act, int64_t max_tiles, in
     a.w = static_cast<const u8 *>(w); a.w2 = static_cast<const u8 *>(w2);
     a.ebytes = fmt_row_bytes(fg, k) * n;
     a.ebytes2 = fmt_row_bytes(fu, k) * n;
-    a.up_off = 0;
     a.n_blocks = (int)((n + 63) / 64);
     a.tiles_m = (int)max_tiles;
     a.tiles_total = (int)max_tiles * a.n_blocks;
@@ -685,26 +567,17 @@ int qmm_grouped_q4k(int fmt, int mode, int fused, int act, int64_t max_tiles, in
     return qmm_grouped_q4k_narrow(0, mode, fused, act, max_tiles, k, n, E, KU, tile_info, rowmap, x, x_scales, x_rows,
                                   w, w2, bias, bias2, y, s);
   const int64_t RB = fmt_row_bytes(fmt, k);
-  Args a{};
-  a.M = (int)(max_tiles * BM); a.N = (int)n; a.K = (int)k;
-  a.x16 = static_cast<const _Float16 *>(x); a.scales = x_scales; a.x_rows = (int)x_rows;
-  a.tile_info = tile_info; a.rowmap = rowmap; a.KU = KU; a.E = E; a.act = act; a.y = y;
-  a.bias = bias; a.bias2 = mode == 0 ? bias2 : nullptr;
-  a.w = static_cast<const u8 *>(w);
-  if (mode == 0) {
-    if (!fused && !w2) return QMM_ERR_NULL;
-    a.ebytes = RB * n * (fused ? 2 : 1);
-    a.ebytes2 = RB * n;
-    a.up_off = fused ? RB * n : 0;
-    a.w2 = fused ? nullptr : static_cast<const u8 *>(w2);
-    a.n_blocks = (int)((n + 63) / 64);
-    a.tiles_m = (int)max_tiles;
-    a.tiles_total = (int)max_tiles * a.n_blocks;
-    return launch_fmt<kGU, false, false>(fmt, a, s);
-  }
-  a.ebytes = RB * n;
-  a.n_blocks = (int)((n + 127) / 128);
-  a.tiles_m = (int)max_tiles;
-  a.tiles_total = (int)max_tiles * a.n_blocks;
-  return launch_fmt<kDN, false, false>(fmt, a, s);
+  if (mode == 0 && !fused && !w2) return QMM_ERR_NULL;
+  TileArgs t{};
+  t.M = (int)(max_tiles * BM); t.N = (int)n; t.K = (int)k;
+  t.x16 = static_cast<const _Float16 *>(x); t.scales = x_scales; t.x_rows = (int)x_rows;
+  t.tile_info = tile_info; t.rowmap = rowmap; t.KU = KU; t.E = E; t.act = act; t.y = y;
+  t.bias = bias; t.bias2 = mode == 0 ? bias2 : nullptr;
+  t.w = static_cast<const u8 *>(w);
+  t.ebytes = RB * n * (mode == 0 && fused ? 2 : 1);
+  t.ebytes2 = RB * n;
+  t.up_off = mode == 0 && fused ? RB * n : 0;
+  t.w2 = mode == 0 && !fused ? static_cast<const u8 *>(w2) : nullptr;
+  t.tiles_m = (int)max_tiles;
+  return tile_gemm(fmt, mode == 0 ? kTGU : kTDN, kT64x4x1, t, s);
 }
