@@ -12,6 +12,8 @@
 //   qmm_row_scale_f16_rows  the same over listed rows (the bucket's pos): the rows g_row_scale_f16_tiles covers
 //   qmm_quant_mxfp8    E4M3 + E8M0-per-32 operand of the scaled MFMA
 //   qmm_repack_mxfp4   GGUF 17-byte MXFP4 blocks -> split planes
+#include <type_traits>
+
 #include "common.hpp"
 #include "topk.hpp"
 
@@ -139,11 +141,14 @@ static void launch_topk(const float *logits, int64_t tokens, int E, int KU, int 
 
 // ------------------------------------------------------------------------------------------------ router
 // out[t, e] = sum_k x[t, k] W[e, k] with fp32 accumulation: the router matvec of g_moe_route[_tr] (S/gen_moe.py:
-// 116-252, :255-460) and, with one row and the sigmoid, g_moe_shared_gate (S/gen_moe.py:780-823). One wave per
-// (row e, group of kRouteTok tokens), row fastest so the waves of a token group share its x rows in L2; lane l
-// reads the 4-value chunks l, l + 64, ... of the row (one 1 KB contiguous piece per wave load for f32 weights)
-// and the same chunks of each token's x. The lane sums its chunks in order, then the butterfly sums the lanes.
-constexpr int kRouteTok = 8;
+// 116-252, :255-460) and, with one row and the sigmoid, g_moe_shared_gate (S/gen_moe.py:780-823). One wave per RE rows
+// e x RT tokens, rows fastest so the waves of a token group share its x rows in L2; lane l reads the 4-value chunks l,
+// l + 64, ... of each row (one 1 KB contiguous piece per wave load for f32 weights) and the same chunks of each token's
+// x. The lane sums its chunks in order, then a butterfly sums the lanes: the same sums whatever RE and RT. A wave of
+// one row and eight tokens loads nine pieces for 32 FMAs a lane, which left a prefill bound by its loads: 8 x 8 loads 16
+// for 256 (1000 tokens x 128 x 2048 with its top-k: 59.8 -> 20.6 us). Few tokens take one row and RT = 1 or 2 with kRouteAhead
+// chunks of every load in flight, for more waves of fewer serial loads (13 tokens: 14.1 -> 7.5 us).
+constexpr int kRouteAhead = 4;
 
 template <bool BF>
 __device__ __forceinline__ f32x4 load4(const void *p, int64_t i4) {
@@ -156,39 +161,85 @@ __device__ __forceinline__ f32x4 load4(const void *p, int64_t i4) {
   }
 }
 
-template <bool XBF, bool WBF>
+// Sums NV values a lane over the wave through the pairing of a butterfly on each value (wave_sum's sums, bit for bit):
+// a step hands half the lane's values to its partner while more than one is left. Returns the value of index `owned`,
+// which lanes with equal lane / (64 / NV) share.
+template <int CNT, int OFF, int NV>
+__device__ __forceinline__ float wave_sum_step(float (&v)[NV], int lane, int &owned) {
+  constexpr int half = CNT / 2;
+  if constexpr (CNT > 1) {
+    const bool up = (lane & OFF) != 0;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      const float send = up ? v[i] : v[half + i], keep = up ? v[half + i] : v[i];
+      v[i] = keep + __shfl_xor(send, OFF, kWave);
+    }
+    owned += up ? half : 0;
+  } else {
+    v[0] += __shfl_xor(v[0], OFF, kWave);
+  }
+  if constexpr (OFF > 1) return wave_sum_step<(CNT > 1 ? half : 1), OFF / 2>(v, lane, owned);
+  else return v[0];
+}
+template <int NV>
+__device__ __forceinline__ float wave_sum_of(float (&v)[NV], int lane, int &owned) {
+  owned = 0;
+  return wave_sum_step<NV, 32>(v, lane, owned);
+}
+
+template <bool XBF, bool WBF, int RT, int RE>
 __global__ __launch_bounds__(256) void router_kernel(int64_t tokens, int64_t H, int E, const void *__restrict__ x,
                                                      const void *__restrict__ w, int sigmoid, float *__restrict__ out) {
+  constexpr int NV = RT * RE;
+  static_assert((NV & (NV - 1)) == 0 && NV <= 64, "wave_sum_of");
   const int lane = threadIdx.x & 63;
   const int64_t gw = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int e = (int)(gw % E);
-  const int64_t t0 = gw / E * kRouteTok;
+  const int eb = (E + RE - 1) / RE;
+  const int e0 = (int)(gw % eb) * RE;
+  const int64_t t0 = gw / eb * RT;
   if (t0 >= tokens) return;
   const int64_t C = H / 4;                 // 4-value chunks of a row
-  int64_t xrow[kRouteTok];
+  int64_t xrow[RT], wrow[RE];
 #pragma unroll
-  for (int r = 0; r < kRouteTok; ++r) xrow[r] = (t0 + r < tokens ? t0 + r : tokens - 1) * C;   // tail: reread
-  float acc[kRouteTok];
+  for (int r = 0; r < RT; ++r) xrow[r] = (t0 + r < tokens ? t0 + r : tokens - 1) * C;   // tail: reread
 #pragma unroll
-  for (int r = 0; r < kRouteTok; ++r) acc[r] = 0.f;
-  const int64_t wrow = (int64_t)e * C;
-#pragma unroll 2
-  for (int64_t c = lane; c < C; c += 64) {
-    const f32x4 wv = load4<WBF>(w, wrow + c);
+  for (int q = 0; q < RE; ++q) wrow[q] = (int64_t)(e0 + q < E ? e0 + q : E - 1) * C;
+  float acc[NV];
 #pragma unroll
-    for (int r = 0; r < kRouteTok; ++r) {
-      const f32x4 xv = load4<XBF>(x, xrow[r] + c);
-      acc[r] = __builtin_fmaf(wv.x, xv.x, acc[r]);
-      acc[r] = __builtin_fmaf(wv.y, xv.y, acc[r]);
-      acc[r] = __builtin_fmaf(wv.z, xv.z, acc[r]);
-      acc[r] = __builtin_fmaf(wv.w, xv.w, acc[r]);
-    }
+  for (int i = 0; i < NV; ++i) acc[i] = 0.f;
+  auto add = [&](const f32x4 (&wv)[RE], const f32x4 (&xv)[RT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int q = 0; q < RE; ++q) acc[r * RE + q] = __builtin_fmaf(wv[q][j], xv[r][j], acc[r * RE + q]);
+  };
+  auto load = [&](f32x4 (&wv)[RE], f32x4 (&xv)[RT], int64_t c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < RE; ++q) wv[q] = load4<WBF>(w, wrow[q] + c);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) xv[r] = load4<XBF>(x, xrow[r] + c);
+  };
+  constexpr int AHEAD = NV >= 64 ? 2 : kRouteAhead;
+  int64_t c = lane;
+  for (; c + 64 * (AHEAD - 1) < C; c += 64 * AHEAD) {
+    f32x4 wv[AHEAD][RE], xv[AHEAD][RT];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) load(wv[u], xv[u], c + 64 * u);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) add(wv[u], xv[u]);
   }
-#pragma unroll
-  for (int r = 0; r < kRouteTok; ++r) {
-    const float v = wave_sum(acc[r]);
-    if (lane == 0 && t0 + r < tokens) out[(t0 + r) * E + e] = sigmoid ? 1.f / (1.f + expf(-v)) : v;
+  for (; c < C; c += 64) {
+    f32x4 wv[RE], xv[RT];
+    load(wv, xv, c);
+    add(wv, xv);
   }
+  int owned;
+  const float v = wave_sum_of<NV>(acc, lane, owned);
+  const int64_t t = t0 + owned / RE;
+  const int e = e0 + owned % RE;
+  if (lane % (64 / NV) == 0 && t < tokens && e < E) out[t * E + e] = sigmoid ? 1.f / (1.f + expf(-v)) : v;
 }
 
 // ------------------------------------------------------------------------------------------------ wscale
@@ -610,8 +661,8 @@ __device__ __forceinline__ void load8(const void *x, int64_t i8, float (&v)[8]) 
 
 // One wave per row (four rows a workgroup): lane l handles the 8-value chunks l, l + 64, ... (NCH of them at most,
 // held in registers between the row maximum and the conversion); the maximum is a wave butterfly, so the row needs no
-// workgroup barrier or LDS. Rows up to 64 x 8 x NCH values; the host takes the scalar kernel above for wider,
-// misaligned or k % 8 != 0 rows.
+// workgroup barrier or LDS. Rows up to 64 x 8 x NCH values; the host takes the workgroup-a-row kernel below
+// for wider rows, the scalar kernel above for misaligned or k % 8 != 0 ones.
 template <bool BF, int NCH>
 __global__ __launch_bounds__(256) void row_scale_wave_kernel(int64_t rows, int64_t k, const void *__restrict__ x,
                                                              float *__restrict__ scales, _Float16 *__restrict__ x16,
@@ -670,6 +721,63 @@ __global__ __launch_bounds__(256) void row_scale_wave_kernel(int64_t rows, int64
     }
   }
   if (lane == 0) {
+    scales[2 * r] = sc;
+    scales[2 * r + 1] = inv;
+  }
+}
+
+// Longer rows: one workgroup per row, thread t the 16-byte pieces t, t + 256, ... of it (NCH at most, held in registers
+// between the maximum and the conversion, all loaded before any is used), so the row is read once where the scalar
+// kernel read it twice, a value a load (2048 x 12288 f32: 42 -> 23 us; bf16 39.5 -> 15.7).
+constexpr int kRsBlockValues = 32768;   // values of the longest row
+template <bool BF, int NCH>
+__global__ __launch_bounds__(256) void row_scale_block_kernel(int64_t k, const void *__restrict__ x,
+                                                              float *__restrict__ scales, _Float16 *__restrict__ x16,
+                                                              const int32_t *__restrict__ tile_info,
+                                                              const int32_t *__restrict__ info) {
+  constexpr int V = BF ? 8 : 4;   // values of a piece
+  const int64_t r = blockIdx.x;
+  if (tile_info && (tile_info[2 * (r / kTile)] < 0 || r % kTile >= tile_info[2 * (r / kTile) + 1])) return;
+  if (pad_row(info, r, k, scales, x16)) return;
+  const int nch = (int)(k / V);
+  const int64_t base = r * nch;
+  v4u q[NCH];
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = (int)threadIdx.x + 256 * i;
+    q[i] = reinterpret_cast<const v4u *>(x)[base + (c < nch ? c : nch - 1)];   // past the row: its last piece again
+  }
+  auto value = [&](int i, int j) {
+    const u32 d = q[i][BF ? j / 2 : j];
+    return BF ? bf16_to_f32(j & 1 ? d >> 16 : d & 0xFFFFu) : u32_as_f32(d);
+  };
+  float m = 0.f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+#pragma unroll
+    for (int j = 0; j < V; ++j) m = fmaxf(m, fabsf(value(i, j)));
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  __shared__ float wmax[4];
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+  const int biased = (int)((f32_as_u32(m) >> 23) & 255u);
+  const int e = min(max(biased - 127 - 13, 0), 100);
+  const float sc = u32_as_f32((u32)(127 - e) << 23), inv = u32_as_f32((u32)(127 + e) << 23);
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = (int)threadIdx.x + 256 * i;
+    if (c >= nch) break;
+    u32 o[V / 2];
+#pragma unroll
+    for (int j = 0; j < V / 2; ++j)
+      o[j] = (u32)__builtin_bit_cast(u16, (_Float16)(value(i, 2 * j) * sc)) |
+             ((u32)__builtin_bit_cast(u16, (_Float16)(value(i, 2 * j + 1) * sc)) << 16);
+    if constexpr (BF) reinterpret_cast<v4u *>(x16)[base + c] = v4u{o[0], o[1], o[2], o[3]};
+    else reinterpret_cast<uint2 *>(x16)[base + c] = make_uint2(o[0], o[1]);
+  }
+  if (threadIdx.x == 0) {
     scales[2 * r] = sc;
     scales[2 * r + 1] = inv;
   }
@@ -804,14 +912,27 @@ static int router(int64_t tokens, int64_t H, int E, const void *x, int x_dtype, 
   if (H <= 0 || H % 4 || H > (1 << 20)) return QMM_ERR_SHAPE;
   const bool xb = x_dtype == QMM_BF16, wb = w_dtype == QMM_BF16;
   if (!aligned(x, xb ? 8 : 16) || !aligned(w, wb ? 8 : 16) || !aligned(out, 4)) return QMM_ERR_ALIGN;
-  const int64_t waves = (int64_t)E * ((tokens + kRouteTok - 1) / kRouteTok);
-  const unsigned grid = (unsigned)((waves + 3) / 4);
+  auto go = [&](auto xc, auto wc, auto rt, auto re) {
+    constexpr int RT = decltype(rt)::value, RE = decltype(re)::value;
+    const int64_t waves = (int64_t)((E + RE - 1) / RE) * ((tokens + RT - 1) / RT);
+    router_kernel<decltype(xc)::value, decltype(wc)::value, RT, RE>
+        <<<(unsigned)((waves + 3) / 4), 256, 0, s>>>(tokens, H, E, x, w, sigmoid, out);
+  };
+  auto shape = [&](auto xc, auto wc) {
+    using std::integral_constant;
+    // 8 x 8 from where its waves fill the chip's 1024 SIMDs (E = 128: 512 tokens), 4 x 4 from a quarter of that
+    const int64_t outs = tokens * E;
+    if (E >= 8 && outs >= 65536) go(xc, wc, integral_constant<int, 8>{}, integral_constant<int, 8>{});
+    else if (E >= 4 && outs >= 8192) go(xc, wc, integral_constant<int, 4>{}, integral_constant<int, 4>{});
+    else if (tokens > 4) go(xc, wc, integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    else go(xc, wc, integral_constant<int, 1>{}, integral_constant<int, 1>{});
+  };
   if (xb) {
-    if (wb) router_kernel<true, true><<<grid, 256, 0, s>>>(tokens, H, E, x, w, sigmoid, out);
-    else router_kernel<true, false><<<grid, 256, 0, s>>>(tokens, H, E, x, w, sigmoid, out);
+    if (wb) shape(std::true_type{}, std::true_type{});
+    else shape(std::true_type{}, std::false_type{});
   } else {
-    if (wb) router_kernel<false, true><<<grid, 256, 0, s>>>(tokens, H, E, x, w, sigmoid, out);
-    else router_kernel<false, false><<<grid, 256, 0, s>>>(tokens, H, E, x, w, sigmoid, out);
+    if (wb) shape(std::false_type{}, std::true_type{});
+    else shape(std::false_type{}, std::false_type{});
   }
   return launch_status();
 }
@@ -913,6 +1034,17 @@ static int row_scale(int64_t rows, int64_t k, const void *x, int x_dtype, float 
     else if (per <= 8) QMM_RS(8);
     else QMM_RS(16);
 #undef QMM_RS
+  } else if (k % 8 == 0 && k <= kRsBlockValues && aligned(x, 16) && aligned(x16, 16)) {
+#define QMM_RSB(BF, N) row_scale_block_kernel<BF, N><<<(unsigned)rows, 256, 0, s>>>(k, x, scales, o, tile_info, info)
+    if (x_dtype == QMM_BF16) {
+      if (k <= 16384) QMM_RSB(true, 8);
+      else QMM_RSB(true, 16);
+    } else {
+      if (k <= 12288) QMM_RSB(false, 12);
+      else if (k <= 16384) QMM_RSB(false, 16);
+      else QMM_RSB(false, 32);
+    }
+#undef QMM_RSB
   } else {
     row_scale_kernel<<<(unsigned)rows, 256, 0, s>>>(rows, k, x, x_dtype == QMM_BF16, scales, o, tile_info, info);
   }
