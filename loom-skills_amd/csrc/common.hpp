@@ -79,6 +79,13 @@ __device__ __forceinline__ float act_fn(int act, float g, float u) {
   return g / (1.0f + expf(-g)) * u;
 }
 
+// Q6_K (210-byte super-blocks, only 2-byte aligned): 16-byte pieces are loaded at any even address (the HSA
+// runtime runs the GPU in unaligned access mode; the compiler emits global_load_dwordx4 for them).
+typedef uint4 uint4_a2 __attribute__((aligned(2)));
+typedef u32 u32_a2 __attribute__((aligned(2)));
+__device__ __forceinline__ uint4 ld16u(const u8 *p) { return *reinterpret_cast<const uint4_a2 *>(p); }
+__device__ __forceinline__ u32 ld4u(const u8 *p) { return *reinterpret_cast<const u32_a2 *>(p); }
+
 // ----------------------------------------------------------------------------------------- wave reductions
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

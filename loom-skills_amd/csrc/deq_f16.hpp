@@ -65,13 +65,6 @@ __device__ __forceinline__ f16x8 deq8_q40(u32 q0, u32 q1, h2 d) {
   return __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
 }
 
-// Q6_K (210-byte super-blocks, only 2-byte aligned): 16-byte pieces are loaded at any even address (the HSA
-// runtime runs the GPU in unaligned access mode; the compiler emits global_load_dwordx4 for them).
-typedef uint4 uint4_a2 __attribute__((aligned(2)));
-typedef u32 u32_a2 __attribute__((aligned(2)));
-__device__ __forceinline__ uint4 ld16u(const u8 *p) { return *reinterpret_cast<const uint4_a2 *>(p); }
-__device__ __forceinline__ u32 ld4u(const u8 *p) { return *reinterpret_cast<const u32_a2 *>(p); }
-
 // f16 (d sc, -dmin m) of sub-block g from a super-block header, broadcast to both halves
 __device__ __forceinline__ void sub_scale(const uint4 &hd, int g, h2 &dsc, h2 &nmn) {
   u32 sc, mn;

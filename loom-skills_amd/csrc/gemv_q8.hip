@@ -118,8 +118,23 @@ __device__ __forceinline__ void xq_load(const u8 *codes, const float *meta, int6
   x.da = u32_as_f32(m.x); x.sa = u32_as_f32(m.y); x.db = u32_as_f32(m.z); x.sb = u32_as_f32(m.w);
 }
 
+// the fragment of an item of 64 values (P::group its first group)
+template <class P>
+struct Item64 {
+  using X = XQ;
+  static constexpr int kAhead = 1;      // passes over a row whose loads are in flight together
+  static constexpr bool kTwoSums = false;
+  static __device__ __forceinline__ void load_x(const u8 *codes, const float *meta, int item, bool live, XQ &x) {
+    xq_load(codes, meta, P::group(item), live, x);
+  }
+  template <class W>
+  static __device__ __forceinline__ float mac(const W &w, const XQ &x, int item, float acc) {
+    return acc + P::dot(w, x, item);
+  }
+};
+
 // Q4_K: item = 4 * block + page j; groups 8 block + 2 j (low nibbles) and + 1 (high nibbles)
-struct Q4K8 {
+struct Q4K8 : Item64<Q4K8> {
   static constexpr bool kSplit = false;
   struct W { v4u h, q0, q1; };
   static __host__ __device__ __forceinline__ int items(int64_t k) { return (int)(k / 256) * 4; }
@@ -152,7 +167,7 @@ struct Q4K8 {
 };
 
 // Q4_0: item = pair of blocks p (36 bytes at 36 p, 4-byte aligned when K % 64 == 0); groups 2 p and 2 p + 1
-struct Q408 {
+struct Q408 : Item64<Q408> {
   static constexpr bool kSplit = false;
   struct W { u32 v[9]; };
   static __host__ __device__ __forceinline__ int items(int64_t k) { return (int)(k / 64); }
@@ -182,39 +197,59 @@ struct Q408 {
   }
 };
 
-// Q6_K: item = 4 b + 2 half + jh (rowdot.hpp q6k_load); groups 2 item (values 0..31) and 2 item + 1. The codes are
+// Q6_K: item = 32 values, 8 b + 4 half + i (i = 0..3): the 16 ql bytes 64 half + 16 i .. of block b, whose low nibbles are
+// values 16 (i % 2) .. + 15 of the half's group i / 2 and whose high nibbles the same values of group i / 2 + 2; qh
+// bytes 32 half + 16 (i % 2) .. . The four lanes of a half read its 64 ql bytes as one piece and the blocks of a wave's
+// 64 lanes are contiguous. (With 64 values a lane every ql byte was loaded by two lanes, 26 dwords an item realigned from
+// even addresses, and the loads' address cycles bound the kernel: 4096 x 12288 at one token 29.6 -> 13 us with its quantizer launch.) The codes are
 // taken unsigned and 32 times the activation code sum of each 16-value run removed, the same integer as the
-// reference's signed codes q - 32 (iq_dot, S/gen_llm.py:1036-1044): per group (ilo s0 + ihi s1) da, s = d sc.
+// reference's signed codes q - 32 (iq_dot, S/gen_llm.py:1036-1044); a run adds (its integer dot) sc da d.
 struct Q6K8 {
   static constexpr bool kSplit = false;
-  using W = Q6W;
-  static __host__ __device__ __forceinline__ int items(int64_t k) { return (int)(k / 256) * 4; }
-  static __device__ __forceinline__ int64_t group(int item) { return 2 * (int64_t)item; }
-  static __device__ __forceinline__ void load_w(const u8 *row, int item, bool live, W &w) {
-    q6k_load(row, item, live, w);
+  static constexpr int kAhead = 3;
+  static constexpr bool kTwoSums = true;   // a lane's even and odd passes summed apart: twice as many passes as with 64
+                                           // values an item, the same rounding
+  struct X { v4u a, b; float da, db; };
+  struct W { uint4 l, h; u32 s0, s1, d; };
+  static __host__ __device__ __forceinline__ int items(int64_t k) { return (int)(k / 256) * 8; }
+  static __device__ __forceinline__ void load_x(const u8 *codes, const float *meta, int item, bool live, X &x) {
+    const int64_t g = (int64_t)(item >> 2) * 4 + ((item >> 1) & 1);   // groups g and g + 2
+    const u8 *c = codes + 32 * g + 16 * (item & 1);
+    const v4u z{0u, 0u, 0u, 0u};
+    x.a = live ? *reinterpret_cast<const v4u *>(c) : z;
+    x.b = live ? *reinterpret_cast<const v4u *>(c + 64) : z;
+    x.da = live ? meta[2 * g] : 0.f;
+    x.db = live ? meta[2 * g + 4] : 0.f;
   }
-  static __device__ __forceinline__ float dot(const W &w, const XQ &x, int item) {
-    u32 ca[8], cb[8];
-    q6k_codes(w, item & 1, ca, cb);
-    float s[4];
-    q6k_scales(w, s);
-    int i16[4];
+  // unconditional (the callers clamp items and rows to real ones, whose x is zero or whose sums are not stored): loads
+  // in branches of their own would be waited for one by one
+  static __device__ __forceinline__ void load_w(const u8 *row, int item, bool, W &w) {
+    const u8 *b = row + (int64_t)(item >> 3) * 210;
+    const int half = (item >> 2) & 1, i = item & 3;
+    w.l = ld16u(b + 64 * half + 16 * i);
+    w.h = ld16u(b + 128 + 32 * half + 16 * (i & 1));
+    w.s0 = ld4u(b + 192 + 8 * half);
+    w.s1 = ld4u(b + 196 + 8 * half);
+    w.d = *reinterpret_cast<const u16 *>(b + 208);
+  }
+  static __device__ __forceinline__ float mac(const W &w, const X &x, int item, float acc) {
+    const int g = (item >> 1) & 1, run = 2 * g + (item & 1);
+    const u32 l[4] = {w.l.x, w.l.y, w.l.z, w.l.w}, h[4] = {w.h.x, w.h.y, w.h.z, w.h.w};
+    const u32 xa[4] = {x.a.x, x.a.y, x.a.z, x.a.w}, xb[4] = {x.b.x, x.b.y, x.b.z, x.b.w};
+    const u32 hs = 2u * (u32)g;
+    int ia = 0, za = 0, ib = 0, zb = 0;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      int ia = 0, za = 0, ib = 0, zb = 0;
-#pragma unroll
-      for (int i = 4 * q; i < 4 * q + 4; ++i) {
-        ia = sdot4(ca[i], x.a[i], ia);
-        za = sdot4(0x20202020u, x.a[i], za);
-        ib = sdot4(cb[i], x.b[i], ib);
-        zb = sdot4(0x20202020u, x.b[i], zb);
-      }
-      i16[q] = ia - za;
-      i16[2 + q] = ib - zb;
+    for (int q = 0; q < 4; ++q) {
+      const u32 hq = h[q] >> hs;   // the group's two high bits in bits 0-1, group + 2's in bits 4-5
+      ia = sdot4((l[q] & 0x0F0F0F0Fu) | ((hq << 4) & 0x30303030u), xa[q], ia);
+      za = sdot4(0x20202020u, xa[q], za);
+      ib = sdot4(((l[q] >> 4) & 0x0F0F0F0Fu) | (hq & 0x30303030u), xb[q], ib);
+      zb = sdot4(0x20202020u, xb[q], zb);
     }
-    const float ga = __builtin_fmaf((float)i16[1], s[1], (float)i16[0] * s[0]) * x.da;
-    const float gb = __builtin_fmaf((float)i16[3], s[3], (float)i16[2] * s[2]) * x.db;
-    return ga + gb;
+    // (integer dot) (8-bit scale) stays below 2^24: exact in f32, so a pair of runs rounds
+    // twice before it joins the sum
+    const int sa = (signed char)((w.s0 >> (8 * run)) & 0xFFu), sb = (signed char)((w.s1 >> (8 * run)) & 0xFFu);
+    return __builtin_fmaf(f16_to_f32(w.d), __builtin_fmaf((float)((ia - za) * sa), x.da, (float)((ib - zb) * sb) * x.db), acc);
   }
 };
 
@@ -249,7 +284,7 @@ __device__ __forceinline__ int e2m1_block_dot(v4u nib, const u32 (&xq)[8]) {
   return acc;
 }
 
-struct MX4S8 {
+struct MX4S8 : Item64<MX4S8> {
   static constexpr bool kSplit = true;
   struct W { v4u a, b; u32 e; };
   static __host__ __device__ __forceinline__ int items(int64_t k) { return (int)(k / 64); }
@@ -304,38 +339,64 @@ __global__ __launch_bounds__(256) void mv_q8_kernel(int64_t n, int64_t tokens, i
     for (int r = 0; r < RL; ++r)
 #pragma unroll
       for (int t = 0; t < TG; ++t) acc[m][r][t] = 0.f;
-  for (int it0 = 0; it0 < nitems; it0 += LPR) {
-    const int item = it0 + sub;
-    const bool live = item < nitems;
-    XQ xs[TG];
+  float alt[NM][RL][TG];   // kTwoSums: the other sum (the two swap places after every pass)
 #pragma unroll
-    for (int t = 0; t < TG; ++t) {
-      const int64_t tok = t0 + t;
-      xq_load(codes + tok * k, meta + 2 * tok * G, P::group(item), live && tok < tokens, xs[t]);
-    }
-    typename P::W wv[NM][RL];
+  for (int m = 0; m < NM; ++m)
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+    for (int r = 0; r < RL; ++r)
 #pragma unroll
-      for (int r = 0; r < RL; ++r) {
-        const int64_t row = row0 + rg + GR * r;
-        load_row<P>((m ? w2 : w) + row * rb, (m ? ws2 : ws) + row * sb, item, live && row < n, wv[m][r]);
+      for (int t = 0; t < TG; ++t) alt[m][r][t] = 0.f;
+  constexpr int UN = RW == 1 ? P::kAhead : 1;
+  for (int it0 = 0; it0 < nitems; it0 += LPR * UN) {
+    typename P::X xs[UN][TG];
+    typename P::W wv[UN][NM][RL];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const bool live = it0 + LPR * u + sub < nitems;
+      const int item = live ? it0 + LPR * u + sub : nitems - 1;
+#pragma unroll
+      for (int t = 0; t < TG; ++t) {
+        const int64_t tok = t0 + t;
+        P::load_x(codes + tok * k, meta + 2 * tok * G, item, live && tok < tokens, xs[u][t]);
       }
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+      for (int m = 0; m < NM; ++m)
 #pragma unroll
-      for (int r = 0; r < RL; ++r)
+        for (int r = 0; r < RL; ++r) {
+          const int64_t row = row0 + rg + GR * r, rc = row < n ? row : n - 1;
+          load_row<P>((m ? w2 : w) + rc * rb, (m ? ws2 : ws) + rc * sb, item, live && row < n, wv[u][m][r]);
+        }
+    }
 #pragma unroll
-        for (int t = 0; t < TG; ++t) acc[m][r][t] += P::dot(wv[m][r], xs[t], item);
+    for (int u = 0; u < UN; ++u) {
+      const bool live = it0 + LPR * u + sub < nitems;
+      const int item = live ? it0 + LPR * u + sub : nitems - 1;
+#pragma unroll
+      for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int r = 0; r < RL; ++r)
+#pragma unroll
+          for (int t = 0; t < TG; ++t) {
+            const float a = P::mac(wv[u][m][r], xs[u][t], item, acc[m][r][t]);
+            if constexpr (P::kTwoSums) {
+              acc[m][r][t] = alt[m][r][t];
+              alt[m][r][t] = a;
+            } else {
+              acc[m][r][t] = a;
+            }
+          }
+    }
   }
 #pragma unroll
   for (int m = 0; m < NM; ++m)
 #pragma unroll
     for (int r = 0; r < RL; ++r)
 #pragma unroll
-      for (int t = 0; t < TG; ++t)
+      for (int t = 0; t < TG; ++t) {
+        if constexpr (P::kTwoSums) acc[m][r][t] += alt[m][r][t];
 #pragma unroll
         for (int off = LPR / 2; off >= 1; off >>= 1) acc[m][r][t] += __shfl_xor(acc[m][r][t], off, kWave);
+      }
   if (sub == 0) {
 #pragma unroll
     for (int r = 0; r < RL; ++r)
@@ -381,6 +442,7 @@ __global__ __launch_bounds__(256) void expert_mv_q8_kernel(int64_t n, int64_t as
   if (row0 >= n || a >= assignments) return;
   const int64_t row = row0 + rr;
   const bool rlive = row < n;
+  const int64_t rclamp = rlive ? row : n - 1;
   int e = ids[a];
   e = e < 0 ? 0 : (e >= E ? E - 1 : e);
   const int64_t xr = GU ? a / KU : a;
@@ -399,15 +461,15 @@ __global__ __launch_bounds__(256) void expert_mv_q8_kernel(int64_t n, int64_t as
 #pragma unroll
   for (int m = 0; m < NM; ++m) acc[m] = 0.f;
   for (int it0 = 0; it0 < nitems; it0 += LPR) {
-    const int item = it0 + sub;
-    const bool live = item < nitems;
-    XQ xs;
-    xq_load(xc, xm, P::group(item), live, xs);
+    const bool live = it0 + sub < nitems;
+    const int item = live ? it0 + sub : nitems - 1;
+    typename P::X xs;
+    P::load_x(xc, xm, item, live, xs);
     typename P::W wv[NM];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) load_row<P>(we[m] + row * rb, se[m] + row * sb, item, live && rlive, wv[m]);
+    for (int m = 0; m < NM; ++m) load_row<P>(we[m] + rclamp * rb, se[m] + rclamp * sb, item, live && rlive, wv[m]);
 #pragma unroll
-    for (int m = 0; m < NM; ++m) acc[m] += P::dot(wv[m], xs, item);
+    for (int m = 0; m < NM; ++m) acc[m] = P::mac(wv[m], xs, item, acc[m]);
   }
 #pragma unroll
   for (int m = 0; m < NM; ++m)
@@ -631,23 +693,35 @@ template <class P, int MODE>
 int launch_generic(int64_t k, int64_t n, int64_t tokens, int accumulate, const void *x, const void *w, const void *w2,
                    int64_t rb, float *y, float *y2, hipStream_t s, const void *ws = nullptr,
                    const void *ws2 = nullptr) {
-  constexpr int TG = 2, RW = MODE == kPlain ? 4 : 2;
   const u8 *codes = static_cast<const u8 *>(x);
   const float *meta = reinterpret_cast<const float *>(codes + tokens * k);
-  const dim3 grid((unsigned)((tokens + TG - 1) / TG), (unsigned)((n + kWaves * RW - 1) / (kWaves * RW)));
-  if (grid.x > 2147483647u || grid.y > 65535u) return QMM_ERR_SHAPE;
   const int items = P::items(k);
-  int lpr = items <= 16 ? 16 : (items <= 32 ? 32 : 64);   // lanes a row, at least 64 / RW
-  lpr = lpr < 64 / RW ? 64 / RW : lpr;
-  auto go = [&](auto lc) {
+  auto go = [&](auto tg, auto rw, auto lc) {
+    constexpr int TG = decltype(tg)::value, RW = decltype(rw)::value;
+    const dim3 grid((unsigned)((tokens + TG - 1) / TG), (unsigned)((n + kWaves * RW - 1) / (kWaves * RW)));
+    if (grid.x > 2147483647u || grid.y > 65535u) return (int)QMM_ERR_SHAPE;
     mv_q8_kernel<P, TG, MODE, RW, decltype(lc)::value><<<grid, 256, 0, s>>>(
         n, tokens, k, accumulate, codes, meta, static_cast<const u8 *>(w), static_cast<const u8 *>(w2), rb,
         static_cast<const u8 *>(ws), static_cast<const u8 *>(ws2), k / 32, y, y2);
     return launch_status();
   };
-  if constexpr (RW >= 4) { if (lpr == 16) return go(std::integral_constant<int, 16>{}); }
-  if (lpr == 32) return go(std::integral_constant<int, 32>{});
-  return go(std::integral_constant<int, 64>{});
+  using std::integral_constant;
+  if constexpr (P::kAhead > 1) {
+    // a row a wave, several passes of loads in flight, while four rows a wave would leave the chip short of waves
+    // (fewer than four a SIMD); its 64 lanes a row give the sums of the narrower maps (their extra lanes hold zeros)
+    if (items > 64 && n * ((tokens + 1) / 2) <= 16384) {
+      if (tokens == 1) return go(integral_constant<int, 1>{}, integral_constant<int, 1>{}, integral_constant<int, 64>{});
+      return go(integral_constant<int, 2>{}, integral_constant<int, 1>{}, integral_constant<int, 64>{});
+    }
+  }
+  constexpr int RW = MODE == kPlain ? 4 : 2;
+  int lpr = items <= 16 ? 16 : (items <= 32 ? 32 : 64);   // lanes a row, at least 64 / RW
+  lpr = lpr < 64 / RW ? 64 / RW : lpr;
+  const integral_constant<int, 2> two;
+  const integral_constant<int, RW> rw;
+  if constexpr (RW >= 4) { if (lpr == 16) return go(two, rw, integral_constant<int, 16>{}); }
+  if (lpr == 32) return go(two, rw, integral_constant<int, 32>{});
+  return go(two, rw, integral_constant<int, 64>{});
 }
 
 template <int MODE>
