@@ -684,6 +684,9 @@ extern "C" int qmm_quant_q8(int64_t rows, int64_t k, const void *x, int x_dtype,
   return launch_status();
 }
 
+bool qmm_mv_q8_mfma_fits(int fmt, int64_t k, int64_t n, int64_t tokens);
+int qmm_mv_q8_mfma(int fmt, int swiglu, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *xq,
+                   const void *w, const void *w2, float *y, hipStream_t s);
 int qmm_mv_q4kt_q8(int fmt, int mode, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *x,
                    int x_dtype, const void *w, const void *w2, float *y, float *y2, hipStream_t s);
 
@@ -752,6 +755,8 @@ extern "C" int qmm_mv_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accu
                          const void *w, float *y, qmm_stream_t stream) {
   if (int st = check_q8(fmt, k, n, tokens, x, x_dtype, w, y)) return st;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (x_dtype == QMM_Q8 && qmm_mv_q8_mfma_fits(fmt, k, n, tokens))
+    return qmm_mv_q8_mfma(fmt, 0, k, n, tokens, accumulate, x, w, nullptr, y, s);
   if (fmt == QMM_Q4_KT || fmt == QMM_Q4_0T)
     return qmm_mv_q4kt_q8(fmt, kPlain, k, n, tokens, accumulate, x, x_dtype, w, nullptr, y, nullptr, s);
   const bool fast = fmt == QMM_Q4_K && (k == 4096 || k == 8192) && tokens <= 65535ll * 2;
@@ -777,6 +782,11 @@ static int mv2_q8(int mode, int fmt, int64_t k, int64_t n, int64_t tokens, int a
   if (!w2 || (mode == kPair && !y2)) return QMM_ERR_NULL;
   if (!aligned(w2, fmt == QMM_Q6_K ? 4 : 16) || (y2 && !aligned(y2, 4))) return QMM_ERR_ALIGN;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (x_dtype == QMM_Q8 && qmm_mv_q8_mfma_fits(fmt, k, n, tokens)) {
+    if (mode == kSwiglu) return qmm_mv_q8_mfma(fmt, 1, k, n, tokens, accumulate, x, w, w2, y, s);
+    if (int st = qmm_mv_q8_mfma(fmt, 0, k, n, tokens, accumulate, x, w, nullptr, y, s)) return st;
+    return qmm_mv_q8_mfma(fmt, 0, k, n, tokens, accumulate, x, w2, nullptr, y2, s);
+  }
   if (fmt == QMM_Q4_KT || fmt == QMM_Q4_0T)
     return qmm_mv_q4kt_q8(fmt, mode, k, n, tokens, accumulate, x, x_dtype, w, w2, y, y2, s);
   if (x_dtype != QMM_Q8) return QMM_ERR_DTYPE;   // GGUF layouts: the planar Q8_1 buffer of qmm_quant_q8

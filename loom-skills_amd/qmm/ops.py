@@ -173,8 +173,9 @@ def _q8_input(fmt, x, k, tokens, staged_tokens):
     tokens = x.shape[0]
     _cols(x, k)
     # the kernels that quantize f32 / bf16 rows themselves do so in every workgroup; from three tokens on a separate
-    # quant_q8 pass is cheaper for the tiled layout (same bits either way)
-    if (fmt == "q4_k" and k in (4096, 8192) and staged_tokens >= 2) or (fmt in TILED_Q8 and tokens <= staged_tokens):
+    # quant_q8 pass is cheaper for the tiled layout (same bits either way), and from nine on the int8 MFMA kernel takes
+    # the planar buffer
+    if (fmt == "q4_k" and k in (4096, 8192) and staged_tokens >= 2 and tokens <= 8) or (fmt in TILED_Q8 and tokens <= staged_tokens):
         return x, _dt(x), tokens
     return quant_q8(x), DTYPE["q8"], tokens
 
