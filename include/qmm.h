@@ -109,7 +109,9 @@ int qmm_quant_q8(int64_t rows, int64_t k, const void *x, int x_dtype, void *xq, 
  * (d da) di with codes q - 8, summed in f32. fmt QMM_Q4_K (k % 256 == 0) or QMM_Q4_0 (k % 64 == 0). x: the planar
  * buffer of qmm_quant_q8 (x_dtype QMM_Q8) for tokens rows, or -- Q4_K with k = 4096 or 8192 only -- f32 / bf16
  * [tokens, k] rows, quantized inside the kernel exactly as qmm_quant_q8 does (same result bit for bit). y: f32
- * [tokens, n]. A multi-token call equals one-token calls bit for bit.
+ * [tokens, n]. A multi-token call equals one-token calls bit for bit, except that Q4_K (either layout) on the planar
+ * buffer runs on the int8 MFMA from 9 tokens and n * tokens >= 32768: the same exact group dots summed in another f32
+ * order (some 1e-7 of the result; the two layouts and the pair call still agree bit for bit there).
  * fmt QMM_Q4_KT: the weights in the tiled layout of qmm_tile_q4k (n % 16 == 0, K % 512 == 0, K / 512 a multiple of
  * at most 4 of a count of at most 8 waves); x planar Q8_1 or f32 / bf16 rows for every such K. For K = 4096 the
  * results equal the QMM_Q4_K call's bit for bit. fmt QMM_Q4_0T: the Q4_0 weights in the tiled layout of qmm_tile_q40,
@@ -130,7 +132,8 @@ int qmm_mv_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accumulate, con
  * kernel there). fmt QMM_Q4_KT / QMM_Q4_0T: W and W2 in the tiled layout of qmm_tile_q4k / qmm_tile_q40, x planar
  * Q8_1 or f32 / bf16 rows
  * (quantized in the kernel exactly as qmm_quant_q8 does); QMM_Q4_K / QMM_Q4_0 / QMM_Q6_K (GGUF): x planar Q8_1.
- * W, W2: [n, k]; y, y2: f32 [tokens, n]. A multi-token call equals one-token calls bit for bit. */
+ * W, W2: [n, k]; y, y2: f32 [tokens, n]. A multi-token call equals one-token calls bit for bit, except as in
+ * qmm_mv_q8. */
 int qmm_mv_swiglu_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *x, int x_dtype,
                      const void *w, const void *w2, float *y, qmm_stream_t stream);
 int qmm_mv_pair_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *x, int x_dtype,

@@ -1,6 +1,6 @@
-// f16 staging of GGUF-block weights for the f16 MFMA kernels, and the expert activation: shared by the prefill GEMM /
-// grouped GEMMs over 64-row tiles (gemm_q4k.hip) and the grouped GEMMs over expert tiles of few rows
-// (grouped_q4k_narrow.hip). The staging is the reference's: Q4_K w = fma_f16(f16(q), f16(d sc), f16(-dmin m))
+// f16 staging of GGUF-block weights for the f16 MFMA kernels, and the expert activation: shared by the tile GEMM
+// (gemm_tile_kernel.hpp), the gate/up pairs in two formats (gemm_q4k.hip) and the grouped GEMMs over expert tiles of few
+// rows (grouped_q4k_narrow.hip). The staging is the reference's: Q4_K w = fma_f16(f16(q), f16(d sc), f16(-dmin m))
 // (S/gen_gemm.py:499-530), Q4_0 w = f16(d (q - 8)) with one rounding (S/moe_q4_0.py:11-38).
 #pragma once
 
@@ -26,11 +26,6 @@ __device__ __forceinline__ f16x8 deq8_codes(u32 n0, u32 n1, h2 dsc, h2 nmn) {
   for (int i = 0; i < 4; ++i) o[i] = as_u32(__builtin_elementwise_fma(as_h2(t[i]) + m1024, dsc, nmn));
   typedef __attribute__((ext_vector_type(4))) u32 u32x4;
   return __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
-}
-template <bool HI>
-__device__ __forceinline__ f16x8 deq8(u32 q0, u32 q1, h2 dsc, h2 nmn) {
-  return deq8_codes(HI ? (q0 >> 4) & 0x0F0F0F0Fu : q0 & 0x0F0F0F0Fu, HI ? (q1 >> 4) & 0x0F0F0F0Fu : q1 & 0x0F0F0F0Fu,
-                    dsc, nmn);
 }
 // The same 8 weights with the codes converted by the FP8 converter: a code byte 0000qqqq read as OCP E4M3 is
 // q 2^-9 exactly, so v_cvt_scalef32_pk_f16_fp8 with scale 512 gives two f16 codes an instruction (where the

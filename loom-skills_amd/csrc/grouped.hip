@@ -1,5 +1,5 @@
 // qmm_moe_grouped: argument checks shared by the grouped expert GEMMs and the dispatch to the GGUF-block (Q4_K, Q6_K,
-// Q4_0: f16 MFMA, gemm_q4k.hip) and MXFP4 split-plane / MFMA-tiled (scaled f8f6f4 MFMA, grouped_mxfp4.hip) kernels.
+// Q4_0: f16 MFMA, by way of gemm_q4k.hip) and MXFP4 split-plane / MFMA-tiled (scaled f8f6f4 MFMA, grouped_mxfp4.hip) kernels.
 // The runtime arguments keep the order of the reference's launches of g_moe_ggu_* / g_moe_gdn_*:
 // (max_rows, k, n, xrows, tile_info, rowmap, x16, scales, w [, w2] [, biases], y) (S/gen_llm.py:5376-5378).
 #include "common.hpp"
@@ -42,7 +42,7 @@ extern "C" int qmm_moe_grouped(int fmt, int mode, int fused, int act, int E, int
   if (mode != 0 && mode != 1) return QMM_ERR_RANGE;
   if (int st = check_grouped(act, E, KU, max_rows, k, n, x_rows, tile_info, rowmap, x, w)) return st;
   if (!y) return QMM_ERR_NULL;
-  // an unfused gate/up needs its up matrix on every kernel path (the narrow and 64-row Q4_K kernels, MXFP4)
+  // an unfused gate/up needs its up matrix on every kernel path (the narrow and tile kernels, MXFP4)
   if (mode == 0 && !fused && !w2) return QMM_ERR_NULL;
   if (mode == 1 && x_rows < max_rows) return QMM_ERR_SHAPE;   // the down GEMM reads its sorted rows in place
   if (!aligned(y, 4) || !aligned(bias, 4) || !aligned(bias2, 4)) return QMM_ERR_ALIGN;

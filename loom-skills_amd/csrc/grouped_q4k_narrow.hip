@@ -1,7 +1,7 @@
 // Grouped expert GEMMs over expert tiles that hold few rows: g_moe_ggu_q4_k[_fused]_k{H} / g_moe_gdn_q4_k_k{FE}
 // (S/gen_moe.py:1126-1228) in the regime where a prefill batch gives each expert a handful of rows (Qwen3-30B-A3B,
-// 64 tokens, top-8 of 128 experts: about four rows an expert). The arithmetic is the 64-row-tile kernel's
-// (gemm_q4k.hip): row-scaled f16 activations, Q4_K weights staged to f16 as fma_f16(f16(q), f16(d sc), f16(-dmin m))
+// 64 tokens, top-8 of 128 experts: about four rows an expert). The arithmetic is the tile GEMM's
+// (gemm_tile_kernel.hpp): row-scaled f16 activations, Q4_K weights staged to f16 as fma_f16(f16(q), f16(d sc), f16(-dmin m))
 // (S/gen_gemm.py:499-530), fp32 accumulation, the row inverse, the expert biases and the activation in the
 // epilogue (S/gen_moe.py:958-1007).
 //

@@ -255,9 +255,15 @@ int launch_nt(const MArgs &a, hipStream_t s) {
 // more, and enough outputs for the grid: 1024 x 4096 at 24 tokens takes 9.4 us here, 9.0 in the matvec kernel; 4096 x 4096
 // 7.9 against 11.9 at nine tokens and 14.4 against 46.6 at 63; 12288 x 4096 gate / up 19.6 against 57.7 and 49 against 287
 // (Q4_K blocks; the tiled layout 17.5 against 36 and 45 against 160).
+// Shapes that the matvec kernels refuse (tiled: a K that does not split over their waves; too many rows) stay theirs.
 bool qmm_mv_q8_mfma_fits(int fmt, int64_t k, int64_t n, int64_t tokens) {
-  return (fmt == QMM_Q4_K || (fmt == QMM_Q4_KT && k % 512 == 0 && n % 16 == 0)) && k % 256 == 0 && tokens >= 9 && n * tokens >= 32768 &&
-         tokens * k < (1ll << 31) && n * (k / 256 * 144) < (1ll << 32) && tokens <= 32 * 65535ll && n <= (1 << 30) - 64;
+  if (fmt != QMM_Q4_K && fmt != QMM_Q4_KT) return false;
+  if (k % 256 || tokens < 9 || n * tokens < 32768 || tokens > 65535 || n > 65535 * 8) return false;
+  if (tokens * k >= (1ll << 31) || n * (k / 256 * 144) >= (1ll << 32)) return false;   // 32-bit byte offsets
+  if (fmt == QMM_Q4_K) return true;
+  bool split = false;   // K = 512 U NW, U <= 4 slices a wave, NW <= 8 waves (qmm_mv_q4kt_q8)
+  for (int u = 1; u <= 4; ++u) split = split || (k / 512 % u == 0 && k / 512 / u <= 8);
+  return n % 16 == 0 && k % 512 == 0 && split;
 }
 
 int qmm_mv_q8_mfma(int fmt, int swiglu, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *xq,
