@@ -109,9 +109,7 @@ int qmm_quant_q8(int64_t rows, int64_t k, const void *x, int x_dtype, void *xq, 
  * (d da) di with codes q - 8, summed in f32. fmt QMM_Q4_K (k % 256 == 0) or QMM_Q4_0 (k % 64 == 0). x: the planar
  * buffer of qmm_quant_q8 (x_dtype QMM_Q8) for tokens rows, or -- Q4_K with k = 4096 or 8192 only -- f32 / bf16
  * [tokens, k] rows, quantized inside the kernel exactly as qmm_quant_q8 does (same result bit for bit). y: f32
- * [tokens, n]. A multi-token call equals one-token calls bit for bit, except that Q4_K (either layout) on the planar
- * buffer runs on the int8 MFMA from 9 tokens and n * tokens >= 32768: the same exact group dots summed in another f32
- * order (some 1e-7 of the result; the two layouts and the pair call still agree bit for bit there).
+ * [tokens, n]. A multi-token call equals one-token calls bit for bit.
  * fmt QMM_Q4_KT: the weights in the tiled layout of qmm_tile_q4k (n % 16 == 0, K % 512 == 0, K / 512 a multiple of
  * at most 4 of a count of at most 8 waves); x planar Q8_1 or f32 / bf16 rows for every such K. For K = 4096 the
  * results equal the QMM_Q4_K call's bit for bit. fmt QMM_Q4_0T: the Q4_0 weights in the tiled layout of qmm_tile_q40,
@@ -127,13 +125,11 @@ int qmm_mv_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accumulate, con
  *   g_mv_{fmt}_k{K}_pair[_t{TG}]_q8[_r{R}], launch args (n, tokens, accumulate, x, w, w2, y, y2):
  *       y[t, r] (+)= g,  y2[t, r] (+)= u
  * with g = x W^T and u = x W2^T computed as qmm_mv_q8 computes one matrix (per 32-value group an exact int32 dot of
- * codes, f32 fixups, the same reductions), so each is bit for bit the one-matrix kernel's of the same layout and K
- * (for GGUF Q4_K at K = 4096 / 8192 that is the tiled layout's, since the one-matrix GGUF call takes its K-sliced
- * kernel there). fmt QMM_Q4_KT / QMM_Q4_0T: W and W2 in the tiled layout of qmm_tile_q4k / qmm_tile_q40, x planar
- * Q8_1 or f32 / bf16 rows
+ * codes, f32 fixups, the same reductions): y and y2 of a pair are bit for bit what qmm_mv_q8 gives, and so are the g and
+ * u of a swiglu except for GGUF Q4_K at K = 4096 / 8192, where the one-matrix call sums in its K-sliced kernel's order.
+ * fmt QMM_Q4_KT / QMM_Q4_0T: W and W2 in the tiled layout of qmm_tile_q4k / qmm_tile_q40, x planar Q8_1 or f32 / bf16 rows
  * (quantized in the kernel exactly as qmm_quant_q8 does); QMM_Q4_K / QMM_Q4_0 / QMM_Q6_K (GGUF): x planar Q8_1.
- * W, W2: [n, k]; y, y2: f32 [tokens, n]. A multi-token call equals one-token calls bit for bit, except as in
- * qmm_mv_q8. */
+ * W, W2: [n, k]; y, y2: f32 [tokens, n]. A multi-token call equals one-token calls bit for bit. */
 int qmm_mv_swiglu_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *x, int x_dtype,
                      const void *w, const void *w2, float *y, qmm_stream_t stream);
 int qmm_mv_pair_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *x, int x_dtype,

@@ -79,6 +79,16 @@ __device__ __forceinline__ float act_fn(int act, float g, float u) {
   return g / (1.0f + expf(-g)) * u;
 }
 
+// Q4_K on Q8_1 activations: the term of a 32-value group before its activation scale, di sc - xs mn (di the exact integer
+// dot, sc = d sc_g, mn = dmin m_g, xs the activation codes' sum), and an item of two groups (terms ta, tb; scales da, db).
+// Written out so that every kernel rounds alike: xs mn rounds first, then the fma; b's product, then the fma with a's.
+__device__ __forceinline__ float q4k_q8_term(int di, float sc, float xs, float mn) {
+  return __builtin_fmaf((float)di, sc, -(xs * mn));
+}
+__device__ __forceinline__ float q4k_q8_item(float ta, float da, float tb, float db) {
+  return __builtin_fmaf(ta, da, tb * db);
+}
+
 // Q6_K (210-byte super-blocks, only 2-byte aligned): 16-byte pieces are loaded at any even address (the HSA
 // runtime runs the GPU in unaligned access mode; the compiler emits global_load_dwordx4 for them).
 typedef uint4 uint4_a2 __attribute__((aligned(2)));

@@ -266,8 +266,8 @@ __global__ __launch_bounds__(kMaxWaves * 64) void mv_q4kt_q8_kernel(int64_t n, i
             p += (sc[m][2 * pg] * md[2 * pg]) * (float)ia;
             p += (sc[m][2 * pg + 1] * md[2 * pg + 1]) * (float)ib;
           } else {
-            p += ((float)ia * sc[m][2 * pg] - ms[2 * pg] * mn[m][2 * pg]) * md[2 * pg];
-            p += ((float)ib * sc[m][2 * pg + 1] - ms[2 * pg + 1] * mn[m][2 * pg + 1]) * md[2 * pg + 1];
+            p = __builtin_fmaf(q4k_q8_term(ia, sc[m][2 * pg], ms[2 * pg], mn[m][2 * pg]), md[2 * pg], p);
+            p = __builtin_fmaf(q4k_q8_term(ib, sc[m][2 * pg + 1], ms[2 * pg + 1], mn[m][2 * pg + 1]), md[2 * pg + 1], p);
           }
         }
         part[m][t] = u == 0 ? p : part[m][t] + p;

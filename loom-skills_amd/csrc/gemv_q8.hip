@@ -19,7 +19,9 @@
 // activations it quantizes them while staging, with the quantizer's own arithmetic, so both input forms give
 // identical results. The generic matvec also streams two matrices of one input: swiglu y = silu(x W^T) (x W2^T)
 // (g_mv_{fmt}_k{K}_swiglu[_t{TG}]_q8) and pair y = x W^T, y2 = x W2^T (g_mv_{fmt}_k{K}_pair[_t{TG}]_q8,
-// S/gen_llm.py:1159-1197), each matrix's rows rounded as the one-matrix kernel rounds them.
+// S/gen_llm.py:1159-1197), each matrix's rows rounded as the one-matrix kernel rounds them; a pair that the one-matrix
+// call takes to the fast path goes there too, a matrix a grid layer. From nine tokens Q4_K runs in mv_q8_mfma.hip, in the
+// same summation orders.
 //
 //   qmm_moe_expert_mv_q8  the decode expert matvecs on Q8_1 activations, g_moe_{gu|dn}_{fmt}[_fused]_q8_k{K}_r{R}
 //                         (S/gen_moe.py:535-727 with iq; the MOE_Q8 default of S/gen_llm.py:5290-5303)
@@ -160,9 +162,8 @@ struct Q4K8 : Item64<Q4K8> {
       ia = sdot4(q[i] & 0x0F0F0F0Fu, x.a[i], ia);
       ib = sdot4((q[i] >> 4) & 0x0F0F0F0Fu, x.b[i], ib);
     }
-    const float ga = ((float)ia * (d * (float)sc0) - x.sa * (dmin * (float)m0)) * x.da;
-    const float gb = ((float)ib * (d * (float)sc1) - x.sb * (dmin * (float)m1)) * x.db;
-    return ga + gb;
+    return q4k_q8_item(q4k_q8_term(ia, d * (float)sc0, x.sa, dmin * (float)m0), x.da,
+                       q4k_q8_term(ib, d * (float)sc1, x.sb, dmin * (float)m1), x.db);
   }
 };
 
@@ -504,7 +505,8 @@ constexpr int kSSlots = QMM_Q8_SLOTS;   // row groups per wave (they share the l
 template <int TG, int KB, bool STAGEQ>
 __global__ __launch_bounds__(kSWaves * 64) void mv_q4k_q8s_kernel(int64_t n, int64_t tokens, int accumulate,
                                                                  const void *__restrict__ x, int bf,
-                                                                 const u8 *__restrict__ w, float *__restrict__ y) {
+                                                                 const u8 *__restrict__ w1, const u8 *__restrict__ w2,
+                                                                 float *__restrict__ y1, float *__restrict__ y2) {
   constexpr int K = KB * 4096, IPR = 4 * KB, RG = 64 / IPR, RW = RG * kSSlots, SLICE = 512 * KB, NG = SLICE / 32;
   constexpr int64_t RB = (int64_t)K / 256 * 144;
   __shared__ __align__(16) u32 xc[kSWaves][TG][SLICE / 4];
@@ -512,6 +514,8 @@ __global__ __launch_bounds__(kSWaves * 64) void mv_q4k_q8s_kernel(int64_t n, int
   __shared__ float red[kSWaves][RW][TG];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const u8 *w = blockIdx.z ? w2 : w1;   // pair: a matrix a grid layer
+  float *y = blockIdx.z ? y2 : y1;
   const int64_t t0 = (int64_t)blockIdx.y * TG;
   const int64_t row0 = (int64_t)blockIdx.x * RW;
   const int r = lane / IPR, it = lane % IPR;
@@ -626,8 +630,8 @@ __global__ __launch_bounds__(kSWaves * 64) void mv_q4k_q8s_kernel(int64_t n, int
         ia = sdot4(Q & 0x0F0F0F0Fu, xa[t][2 * pg][i], ia);
         ib = sdot4((Q >> 4) & 0x0F0F0F0Fu, xa[t][2 * pg + 1][i], ib);
       }
-      p += ((float)ia * sc[2 * pg] - ms[t][2 * pg] * mn[2 * pg]) * md[t][2 * pg];
-      p += ((float)ib * sc[2 * pg + 1] - ms[t][2 * pg + 1] * mn[2 * pg + 1]) * md[t][2 * pg + 1];
+      p = __builtin_fmaf(q4k_q8_term(ia, sc[2 * pg], ms[t][2 * pg], mn[2 * pg]), md[t][2 * pg], p);
+      p = __builtin_fmaf(q4k_q8_term(ib, sc[2 * pg + 1], ms[t][2 * pg + 1], mn[2 * pg + 1]), md[t][2 * pg + 1], p);
     }
     // the row's IPR lanes of this slice: a butterfly leaves the slice sum in every one of them
     p += xshfl<1>(p);
@@ -654,21 +658,29 @@ __global__ __launch_bounds__(kSWaves * 64) void mv_q4k_q8s_kernel(int64_t n, int
   }
 }
 
+// one matrix, or a pair (y2)
+struct SArgs {
+  int64_t n, tokens;
+  int accumulate;
+  const void *x;
+  int bf;
+  const void *w, *w2;
+  float *y, *y2;
+};
 template <int TG, int KB, bool STAGEQ>
-int launch_sliced(int64_t n, int64_t tokens, int accumulate, const void *x, int bf, const void *w, float *y,
-                  hipStream_t s) {
+int launch_sliced(const SArgs &a, hipStream_t s) {
   constexpr int RW = 16 / KB * kSSlots;
-  const dim3 grid((unsigned)((n + RW - 1) / RW), (unsigned)((tokens + TG - 1) / TG));
-  mv_q4k_q8s_kernel<TG, KB, STAGEQ><<<grid, kSWaves * 64, 0, s>>>(n, tokens, accumulate, x, bf,
-                                                                  static_cast<const u8 *>(w), y);
+  const dim3 grid((unsigned)((a.n + RW - 1) / RW), (unsigned)((a.tokens + TG - 1) / TG), a.y2 ? 2u : 1u);
+  mv_q4k_q8s_kernel<TG, KB, STAGEQ><<<grid, kSWaves * 64, 0, s>>>(a.n, a.tokens, a.accumulate, a.x, a.bf,
+                                                                  static_cast<const u8 *>(a.w),
+                                                                  static_cast<const u8 *>(a.w2), a.y, a.y2);
   return launch_status();
 }
 
-template <int KB, bool STAGEQ>
-int launch_fast_tg(int64_t n, int64_t tokens, int accumulate, const void *x, int bf, const void *w, float *y,
-                   hipStream_t s) {
-  return tokens >= 2 ? launch_sliced<2, KB, STAGEQ>(n, tokens, accumulate, x, bf, w, y, s)
-                     : launch_sliced<1, KB, STAGEQ>(n, tokens, accumulate, x, bf, w, y, s);
+template <bool STAGEQ>
+int launch_fast(int64_t k, const SArgs &a, hipStream_t s) {
+  if (k == 4096) return a.tokens >= 2 ? launch_sliced<2, 1, STAGEQ>(a, s) : launch_sliced<1, 1, STAGEQ>(a, s);
+  return a.tokens >= 2 ? launch_sliced<2, 2, STAGEQ>(a, s) : launch_sliced<1, 2, STAGEQ>(a, s);
 }
 
 }  // namespace
@@ -685,8 +697,8 @@ extern "C" int qmm_quant_q8(int64_t rows, int64_t k, const void *x, int x_dtype,
 }
 
 bool qmm_mv_q8_mfma_fits(int fmt, int64_t k, int64_t n, int64_t tokens);
-int qmm_mv_q8_mfma(int fmt, int swiglu, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *xq,
-                   const void *w, const void *w2, float *y, hipStream_t s);
+int qmm_mv_q8_mfma(int fmt, int swiglu, int sliced, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *xq,
+                   const void *w, const void *w2, float *y, float *y2, hipStream_t s);
 int qmm_mv_q4kt_q8(int fmt, int mode, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *x,
                    int x_dtype, const void *w, const void *w2, float *y, float *y2, hipStream_t s);
 
@@ -749,28 +761,28 @@ int check_q8(int fmt, int64_t k, int64_t n, int64_t tokens, const void *x, int x
   if (!aligned(x, 16) || !aligned(w, fmt == QMM_Q6_K ? 4 : 16) || !aligned(y, 4)) return QMM_ERR_ALIGN;
   return QMM_OK;
 }
+// the one-matrix Q4_K calls of the K-sliced kernel (GGUF blocks)
+bool sliced_call(int fmt, int64_t k, int64_t tokens) {
+  return fmt == QMM_Q4_K && (k == 4096 || k == 8192) && tokens <= 65535ll * 2;
+}
 }  // namespace
 
 extern "C" int qmm_mv_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *x, int x_dtype,
                          const void *w, float *y, qmm_stream_t stream) {
   if (int st = check_q8(fmt, k, n, tokens, x, x_dtype, w, y)) return st;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const bool fast = sliced_call(fmt, k, tokens);
   if (x_dtype == QMM_Q8 && qmm_mv_q8_mfma_fits(fmt, k, n, tokens))
-    return qmm_mv_q8_mfma(fmt, 0, k, n, tokens, accumulate, x, w, nullptr, y, s);
+    return qmm_mv_q8_mfma(fmt, 0, fast, k, n, tokens, accumulate, x, w, nullptr, y, nullptr, s);
   if (fmt == QMM_Q4_KT || fmt == QMM_Q4_0T)
     return qmm_mv_q4kt_q8(fmt, kPlain, k, n, tokens, accumulate, x, x_dtype, w, nullptr, y, nullptr, s);
-  const bool fast = fmt == QMM_Q4_K && (k == 4096 || k == 8192) && tokens <= 65535ll * 2;
+  const SArgs a{n, tokens, accumulate, x, x_dtype == QMM_BF16, w, nullptr, y, nullptr};
   if (x_dtype != QMM_Q8) {
     // f32 / bf16 rows are quantized while staged; only the fast path stages (others take planar Q8 from
     // qmm_quant_q8)
-    if (!fast) return QMM_ERR_SHAPE;
-    const int bf = x_dtype == QMM_BF16;
-    return k == 4096 ? launch_fast_tg<1, true>(n, tokens, accumulate, x, bf, w, y, s)
-                     : launch_fast_tg<2, true>(n, tokens, accumulate, x, bf, w, y, s);
+    return fast ? launch_fast<true>(k, a, s) : QMM_ERR_SHAPE;
   }
-  if (fast)
-    return k == 4096 ? launch_fast_tg<1, false>(n, tokens, accumulate, x, 0, w, y, s)
-                     : launch_fast_tg<2, false>(n, tokens, accumulate, x, 0, w, y, s);
+  if (fast) return launch_fast<false>(k, a, s);
   return generic_fmt<kPlain>(fmt, k, n, tokens, accumulate, x, w, nullptr, y, nullptr, s);
 }
 
@@ -783,13 +795,15 @@ static int mv2_q8(int mode, int fmt, int64_t k, int64_t n, int64_t tokens, int a
   if (!aligned(w2, fmt == QMM_Q6_K ? 4 : 16) || (y2 && !aligned(y2, 4))) return QMM_ERR_ALIGN;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (x_dtype == QMM_Q8 && qmm_mv_q8_mfma_fits(fmt, k, n, tokens)) {
-    if (mode == kSwiglu) return qmm_mv_q8_mfma(fmt, 1, k, n, tokens, accumulate, x, w, w2, y, s);
-    if (int st = qmm_mv_q8_mfma(fmt, 0, k, n, tokens, accumulate, x, w, nullptr, y, s)) return st;
-    return qmm_mv_q8_mfma(fmt, 0, k, n, tokens, accumulate, x, w2, nullptr, y2, s);
+    if (mode == kSwiglu) return qmm_mv_q8_mfma(fmt, 1, 0, k, n, tokens, accumulate, x, w, w2, y, nullptr, s);
+    return qmm_mv_q8_mfma(fmt, 0, sliced_call(fmt, k, tokens), k, n, tokens, accumulate, x, w, w2, y, y2, s);
   }
   if (fmt == QMM_Q4_KT || fmt == QMM_Q4_0T)
     return qmm_mv_q4kt_q8(fmt, mode, k, n, tokens, accumulate, x, x_dtype, w, w2, y, y2, s);
   if (x_dtype != QMM_Q8) return QMM_ERR_DTYPE;   // GGUF layouts: the planar Q8_1 buffer of qmm_quant_q8
+  // a pair takes the one-matrix call's kernel, so that its rows are that call's bit for bit
+  if (mode == kPair && sliced_call(fmt, k, tokens) && n <= 65535ll * 8)
+    return launch_fast<false>(k, SArgs{n, tokens, accumulate, x, 0, w, w2, y, y2}, s);
   return mode == kSwiglu ? generic_fmt<kSwiglu>(fmt, k, n, tokens, accumulate, x, w, w2, y, nullptr, s)
                          : generic_fmt<kPair>(fmt, k, n, tokens, accumulate, x, w, w2, y, y2, s);
 }

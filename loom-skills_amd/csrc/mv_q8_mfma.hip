@@ -1,28 +1,42 @@
-// Decode matvecs on Q8_1 activations for 9 tokens and more (Q4_K, GGUF or tiled): g_mv_{fmt}_k{K}[_swiglu]_q8 of a
+// Decode matvecs on Q8_1 activations for 9 tokens and more (Q4_K, GGUF or tiled): g_mv_{fmt}_k{K}[_swiglu|_pair]_q8 of a
 // batch of decoding sequences (S/gen_llm.py:1159-1197, :1288-1301), on the int8 MFMA.
 //
 //   y[t, r] (+)= sum over 32-value groups g of (di sc - xs mn) da,   di = sum q_w q_x (exact), sc = d sc_g,
 //                                                                     mn = dmin m_g, (da, xs) the group's Q8_1 pair
-//   swiglu: y (+)= silu(gate) up
+//   swiglu: y (+)= silu(gate) up;  pair: y (+)= x W^T, y2 (+)= x W2^T (one launch, a matrix a grid layer)
 //
-// The matvec kernels read every weight once per two tokens (GGUF) or eight (tiled) and spend a v_dot4 per four products;
-// 24 tokens through 2 x 12288 x 4096 took 122 us, against 7 us of weight bytes (here 26.5). Here a weight is read once per 32 tokens
-// and 16 x 16 products of a group take one v_mfma_i32_16x16x32_i8 a wave: what is left is the fixup of each group's
-// 256 sums (convert, scale, fma: 12 vector instructions a wave), which bounds it. The codes are taken as 16 (q - 8), so
-// a group adds (16 di - 128 xs) (sc / 16) da - xs (mn - 8 sc) da: the first sums are free of the codes' common offset (with
-// unsigned codes the two terms cancel, and the result was twice as far from 64 bits), and the second term,
-// small, is a product of f32 matrices over the groups: two v_mfma_f32_16x16x4_f32 a super-block.
+// Every output has the bits of the same token's call with fewer tokens (a multi-token call equals one-token calls,
+// make_kernel_tests.py:264-268): di is an exact integer, a group's term takes the roundings of q4k_q8_term (xs mn as a
+// product of one MFMA step, so rounded once, then one fma), and the terms meet in the tree of the kernel that takes the
+// call at one token:
+//   kItems   (gemv_q8.hip, the item walk: every GGUF call but the next) an item is a page, two groups; item lane l sums
+//            page l % 4 of super-blocks l / 4, l / 4 + 16, ..., then the 64 lanes meet in a butterfly (xor 32 .. 1)
+//   kSlices  (gemv_q4kt.hip; gemv_q8.hip's K-sliced kernel, GGUF at K = 4096 / 8192) a wave's slice of K: chains of four
+//            groups (half a super-block) are summed over the units of the slice (tiled), the halves in a butterfly, the
+//            slices in order
 //
-// A workgroup: 16 weight rows (swiglu: 16 of each matrix) x 16 NT tokens, kWaves waves. Wave v takes super-blocks v,
-// v + kWaves, ... of all rows: it brings the super-block's codes and pairs of its tokens into registers (coalesced through its own
-// LDS: a load in which every lane reads its own token or row takes the address unit 64 cycles), then streams the
-// super-block of the rows past them. The waves' sums meet in LDS at the end, in wave order.
+// The matvec kernels read every weight once per two tokens (GGUF) or eight (tiled) and spend a v_dot4 per four products.
+// Here a weight is read once per 16 tokens and 16 x 16 products of a group take one v_mfma_i32_16x16x32_i8 a wave: what is
+// left is the fixup of each group's 256 sums (convert, two fma; kItems half a multiply and half an add more: 12 - 14 vector
+// instructions of a wave's 33 a group), which bounds it: at 48 tokens through 2 x 12288 x 4096 the vector pipes are busy
+// 79 % of the time a CU holds a wave. 24 tokens through it 111 -> 36 us with the quantizer's launch (8 us of weights).
+//
+// A workgroup: 16 weight rows x 16 tokens, eight waves (swiglu: the gate matrix, then the up matrix). A wave takes whole
+// super-blocks of all rows (kItems: v, v + 16, ... and then v + 8, v + 24, ...; kSlices: slice v): it brings the
+// super-block's codes and pairs of its tokens into its own LDS (coalesced: a load in which every lane reads its own token
+// takes the address unit 64 cycles), then the rows' super-block past them, the next one's loads in flight. The waves' sums
+// meet in LDS at the end. That takes up to 128 registers, so four waves a SIMD. Measured and slower at 24 tokens through
+// 2 x 12288 x 4096 (35.7 us): 32 tokens a workgroup (36.4 at two waves a SIMD; at four it spills), half super-blocks
+// (41.7), the gate's meeting before the up matrix (38.4), workgroups that stay for several tiles (38.7).
 //
 // MFMA operands: lane (c, q) = (lane % 16, lane / 16) holds 8 K values of weight row / token c; which 8 does not matter
 // while both agree. A page's 32 code bytes are two groups (low and high nibbles). Lane (c, q) loads bytes 16 q .. of two
 // pages (64 bytes of a row from four lanes); exchanging register halves between lanes 0-31 and 32-63 (v_permlane32_swap)
 // leaves bytes 16 (q % 2) + 8 (q / 2) .. + 7 of the one page in the first two registers and of the other in the last
 // two. A token's 64 codes of a page's two groups go through the same exchange, so they meet the weights at the same K.
+// The sums of 16 tokens x 16 rows lie in four registers: lane (c, q), register i is token 4 q + i, row c, so that a row's
+// scale is one register. The products xs mn of four groups are the four blocks of a v_mfma_f32_16x16x1_4b_f32: lane (c, q)
+// holds row / token c of group q, and register 4 b + i of the result is block b's.
 #include "common.hpp"
 
 using namespace qmm;
@@ -31,249 +45,294 @@ namespace {
 
 typedef __attribute__((ext_vector_type(4))) u32 u32x4;
 
+enum Order { kItems = 0, kSlices = 1 };
+constexpr int kWaves = 8;
 
 struct MArgs {
   int n, tokens, nsb;           // rows of a matrix, tokens, super-blocks a row
+  int tiles;                    // of 16 tokens
+  int chains, units;            // kSlices: slice v is super-blocks v chains units .. ; chain j sums units of them, two apart
   const u8 *codes;              // planar Q8_1: codes [tokens][K], then pairs f32 [tokens][K / 32][2]
   const float *meta;
-  const u8 *w, *w2;
-  float *y;
+  const u8 *w, *w2;             // swiglu: gate, up; pair: the matrices of blockIdx.y = 0 and 1
+  float *y, *y2;
   int accumulate;
 };
 
-// registers (a, b) of a 16-byte piece: halves of the wave exchanged so that a belongs to one page, b to the other
-__device__ __forceinline__ void page_swap(u32 &a, u32 &b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  a = r[0];
-  b = r[1];
+// a 16-byte piece's registers (0, 2) and (1, 3): halves of the wave exchanged so that 0 and 1 belong to one page, 2 and 3
+// to the other
+__device__ __forceinline__ u32x4 page_swap(u32x4 v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+  return u32x4{a[0], b[0], a[1], b[1]};
 }
 __device__ __forceinline__ long pack8(u32 a, u32 b) { return (long)(((uint64_t)b << 32) | a); }
 
-template <bool TL, bool SWIGLU, int NT, int kRowBlocks, int kWaves>
-__global__ __launch_bounds__(64 * kWaves, kWaves == 8 ? 4 : 3) void mv_q8_mfma_kernel(MArgs a) {
-  // LDS bytes a wave: the codes of 16 tokens, per 16 tokens da and xs da [group][token], d sc of 16 rows [group][row]
-  constexpr int kCode = 16 * 256, kMeta = NT * 1024, kScale = 8 * 16 * 4;
-  constexpr int kOwn = kCode + kMeta + kScale;
-  constexpr int kPair = kRowBlocks > 1 ? 2 : 1;                           // row blocks that meet in LDS at a time
-  constexpr int kRed = kPair * NT * 256 * 4;
-  __shared__ __align__(16) u8 smem[kWaves * (kOwn > kRed ? kOwn : kRed)];
+// LONG (kItems): more than 16 super-blocks, so an item lane sums several
+template <bool TL, bool SWIGLU, int ORDER, bool LONG>
+__global__ __launch_bounds__(64 * kWaves, 4) void mv_q8_mfma_kernel(MArgs a) {
+  constexpr int NV = ORDER == kItems ? 4 : 2;                             // sums of a super-block: pages, or halves
+  // LDS bytes a wave: the codes of 16 tokens, their da and xs [group][token]
+  constexpr int kCode = 16 * 256, kMeta = 1024;
+  constexpr int kOwn = kCode + kMeta;
+  static_assert(kOwn >= 4 * 256 * 4, "a wave's share of the meeting");
+  // swiglu: the gate's meeting has its own room
+  __shared__ __align__(16) u8 smem[kWaves * (kOwn + (SWIGLU ? (ORDER == kItems ? 4 : 1) * 256 * 4 : 0))];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, q = lane >> 4;
   const u32 K = (u32)a.nsb * 256u, RB = (u32)a.nsb * 144u;   // all byte offsets fit 32 bits (qmm_mv_q8_mfma_fits)
-  constexpr int kOut = 16 * (SWIGLU ? kRowBlocks / 2 : kRowBlocks);       // output rows a workgroup
-  const int row0 = (int)blockIdx.x * kOut, t0 = (int)blockIdx.y * 16 * NT;
+  // workgroup b runs on XCD b % 8: the token tiles of a row block follow each other there and share its weights in L2
+  const int bi = (int)(blockIdx.x >> 3);
+  const int row0 = ((bi / a.tiles) * 8 + (int)(blockIdx.x & 7)) * 16, t0 = bi % a.tiles * 16;
+  if (row0 >= a.n) return;
+  constexpr bool kAheadX = !LONG;   // the next super-block's tokens too: LONG would spill
   u8 *own = smem + wave * kOwn;
+  float *md = reinterpret_cast<float *>(own + kCode);
 
-  // the lane's row of each row block (rows past n read row n - 1 and are not stored)
-  u32 wr[kRowBlocks];   // byte offset in its matrix
+  // byte offset of the lane's row in its matrix (rows past n read row n - 1 and are not stored); tiled: the lane's plane q
+  // of its 16-row block (the header lies 512 + 1024 q + 32 (row % 16) before it; n % 16 == 0, so row % 16 = c)
+  const int row = min(row0 + c, a.n - 1);
+  const u32 wr = TL ? (u32)(row >> 4) * 16u * RB + 512u + 1024u * (u32)q + 64u * (u32)(row & 15) : (u32)row * RB;
+  const u32 hoff = 512u + 1024u * (u32)q + 32u * (u32)c;
+
+  // ---- the wave's super-blocks in order, the next one's weights and tokens loaded while one is summed
+  struct Pos { int r, sb, j, u; };   // matrix, super-block; kItems: j = 0 (v, v + 16, ..) or 1 (v + 8, ..); kSlices: chain, unit
+  constexpr int kMats = SWIGLU ? 2 : 1;
+  const int per = a.chains * a.units;   // kSlices: super-blocks of a slice
+  const int first = ORDER == kItems ? wave : wave * per;
+  auto next = [&](Pos p) __attribute__((always_inline)) {
+    if constexpr (ORDER == kItems) {
+      p.sb += 2 * kWaves;
+      if (p.sb >= a.nsb && p.j == 0 && wave + kWaves < a.nsb) { p.j = 1; p.sb = wave + kWaves; }
+    } else {
+      if (++p.u == a.units) { p.u = 0; ++p.j; }
+      p.sb = p.j == a.chains ? a.nsb : first + p.j + 2 * p.u;
+    }
+    if (p.sb >= a.nsb) p = Pos{p.r + 1, first, 0, 0};
+    return p;
+  };
+  u32x4 c0, c1, h, v[4], pr;
+  auto load_w = [&](Pos at) __attribute__((always_inline)) {
+    const bool second = SWIGLU ? at.r != 0 : blockIdx.y != 0;
+    const u8 *m = second ? a.w2 : a.w;
+    if constexpr (TL) {
+      // unit sb / 2 (4608 bytes): page p's bytes 16 h .. in plane 2 (p % 2) + h, at 64 row + 32 (sb % 2) + 16 (p / 2);
+      // lane q reads page q / 2 (and 2 + q / 2), half q % 2: plane q
+      const u8 *u = m + (int64_t)(at.sb >> 1) * 4608;
+      c0 = *reinterpret_cast<const u32x4 *>(u + 32 * (at.sb & 1) + wr);
+      c1 = *reinterpret_cast<const u32x4 *>(u + 32 * (at.sb & 1) + 16 + wr);
+      h = *reinterpret_cast<const u32x4 *>(u + 16 * (at.sb & 1) + (wr - hoff));
+    } else {
+      const u8 *b = m + (int64_t)at.sb * 144;
+      c0 = *reinterpret_cast<const u32x4 *>(b + 16 + (wr + 16u * (u32)q));
+      c1 = *reinterpret_cast<const u32x4 *>(b + 80 + (wr + 16u * (u32)q));
+      h = *reinterpret_cast<const u32x4 *>(b + wr);
+    }
+  };
+  auto load_x = [&](Pos at) __attribute__((always_inline)) {
 #pragma unroll
-  for (int r = 0; r < kRowBlocks; ++r) {
-    const bool up = SWIGLU && r >= kRowBlocks / 2;   // swiglu: gate blocks, then their up blocks
-    const int row = min(row0 + 16 * (up ? r - kRowBlocks / 2 : r) + c, a.n - 1);
-    // tiled: the lane's plane q of its 16-row block (the header lies 512 + 1024 q + 32 (row % 16) before it)
-    wr[r] = TL ? (u32)(row >> 4) * 16u * RB + 512u + 1024u * (u32)q + 64u * (u32)(row & 15) : (u32)row * RB;
+    for (int i = 0; i < 4; ++i) {   // 16 lanes a token: its 256 codes
+      const int tok = min(t0 + 4 * i + q, a.tokens - 1);
+      v[i] = *reinterpret_cast<const u32x4 *>(a.codes + at.sb * 256 + ((u32)tok * K + 16u * (u32)c));
+    }
+    const int tok = min(t0 + (lane >> 2), a.tokens - 1);   // four lanes a token: its 8 pairs
+    pr = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const u8 *>(a.meta) + at.sb * 64 +
+                                          ((u32)tok * (K / 4u) + 16u * (u32)(lane & 3)));
+  };
+
+  f32x4 sum[NV], held[NV];   // kItems: held the first class's (LONG); kSlices: held[0] a pair of chains, held[1] the slice
+#pragma unroll
+  for (int i = 0; i < NV; ++i) sum[i] = held[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float *meet = reinterpret_cast<float *>(smem);                      // [wave][NM][token][row]
+  float *meet_gate = reinterpret_cast<float *>(smem + kWaves * kOwn);
+  constexpr int NM = ORDER == kItems ? 4 : 1;                         // sums a wave hands on
+  auto hand = [&](float *to) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NM; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) to[(wave * NM + i) * 256 + 16 * (4 * q + j) + c] = ORDER == kItems ? sum[i][j] : held[1][j];
+  };
+
+  Pos at{first < a.nsb ? 0 : kMats, first, 0, 0};
+  if (SWIGLU && at.r == kMats) hand(meet_gate);   // no super-block: zeros
+  if (at.r < kMats) {
+    load_w(at);
+    load_x(at);
   }
-  const u32 hoff = 512u + 1024u * (u32)q + 32u * (u32)c;   // tiled: rows of a block are the lanes c (row0 % 16 = 0)
-  constexpr bool kTwoSums = !SWIGLU && NT == 1;   // a wave's even and odd super-blocks summed apart, where registers allow
-  f32x4 acc[kRowBlocks][NT], alt[kRowBlocks][NT];
+#pragma unroll 1
+  while (at.r < kMats) {
+    const Pos nx = next(at);
+    // piece i of token k at i ^ k: the 16 tokens of a read lie in different banks
 #pragma unroll
-  for (int r = 0; r < kRowBlocks; ++r)
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x4 *>(own + (4 * i + q) * 256 + 16 * (c ^ (4 * i + q))) = v[i];
+    float *mt = md + 32 * (lane & 3) + (lane >> 2);   // groups 2 (lane % 4) and + 1, token lane / 4
+    mt[0] = u32_as_f32(pr.x);
+    mt[16] = u32_as_f32(pr.z);
+    mt[128] = u32_as_f32(pr.y);
+    mt[144] = u32_as_f32(pr.w);
+    // row c's minima of groups q and q + 4, and its 8 scales (ggml get_scale_min_k4)
+    const u32 sh = 8u * (u32)q;
+    const u32 hz = h.z >> sh, hw = h.w >> sh;
+    const float d = f16_to_f32(h.x), dmin = f16_to_f32(h.x >> 16);
+    const float mn[2] = {dmin * (float)(hz & 63u), dmin * (float)(((hw >> 4) & 15u) | ((hz >> 2) & 48u))};
+    const u32 sc[2] = {h.y & 0x3F3F3F3Fu, (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u)};
+    const u32x4 wq[2] = {page_swap(c0), page_swap(c1)};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (nx.r < kMats) {
+      load_w(nx);
+      if (kAheadX) load_x(nx);
+    }
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[r][t] = alt[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int hf = 0; hf < 2; ++hf) {
+      // -xs mn of groups 4 hf .. 4 hf + 3 where their sums lie: xs of token c, mn of row c, group 4 hf + q
+      const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      const f32x16 xm = __builtin_amdgcn_mfma_f32_16x16x1f32(md[128 + 64 * hf + 16 * q + c], -mn[hf], zero16, 0, 0, 0);
+      f32x4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int pi = 0; pi < 2; ++pi) {   // page p: groups 2 p (low nibbles) and 2 p + 1
+        const int p = 2 * hf + pi;
+        const u32x4 x = page_swap(*reinterpret_cast<const u32x4 *>(own + c * 256 + 16 * ((4 * p + q) ^ c)));
+        f32x4 term[2], da[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          da[e] = *reinterpret_cast<const f32x4 *>(md + 16 * (2 * p + e) + 4 * q);   // of tokens 4 q .. 4 q + 3
+          const float s = d * (float)((sc[hf] >> (8 * (2 * pi + e))) & 0xFFu);
+          const u32 b0 = pi ? wq[hf].z : wq[hf].x, b1 = pi ? wq[hf].w : wq[hf].y;
+          const long wa = pack8((b0 >> (4 * e)) & 0x0F0F0F0Fu, (b1 >> (4 * e)) & 0x0F0F0F0Fu);
+          const long xa = e ? pack8(x.z, x.w) : pack8(x.x, x.y);
+          const i32x4 di = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa, wa, i32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) term[e][i] = __builtin_fmaf((float)di[i], s, xm[8 * pi + 4 * e + i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (ORDER == kItems) {
+            sum[p][i] += q4k_q8_item(term[0][i], da[0][i], term[1][i], da[1][i]);
+          } else {
+            part[i] = __builtin_fmaf(term[0][i], da[0][i], part[i]);
+            part[i] = __builtin_fmaf(term[1][i], da[1][i], part[i]);
+          }
+        }
+      }
+      if constexpr (ORDER == kSlices) sum[hf] += part;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if constexpr (ORDER == kItems) {
+      // item lanes 4 v + p and 4 (v + 8) + p meet, the butterfly's first step (!LONG: one super-block each, the second
+      // joins the first by itself)
+      if (LONG && nx.j != at.j) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          if (at.j == 0) { held[p] = sum[p]; sum[p] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+          else sum[p] += held[p];
+        }
+      }
+    } else if (nx.j != at.j) {   // a chain is done, its halves' sum: (chain 0 + chain 1) + (chain 2 + chain 3)
+      const f32x4 one = sum[0] + sum[1];
+      sum[0] = sum[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      held[0] = at.j & 1 ? held[0] + one : one;
+      if (at.j == 1) held[1] = held[0];
+      if (at.j == 3) held[1] += held[0];
+    }
+    if (SWIGLU && nx.r == 1 && at.r == 0) {
+      hand(meet_gate);
+      if constexpr (ORDER == kItems) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) sum[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    if (!kAheadX && nx.r < kMats) load_x(nx);
+    at = nx;
+  }
 
-  for (int sb = wave; sb < a.nsb; sb += kWaves) {
-    // ---- the super-block's weights of the first row block, then the tokens
-    uint4 c0[2], c1[2], hd[2];
-    auto load_w = [&](int r) __attribute__((always_inline)) {
-      const u8 *m = SWIGLU && r >= kRowBlocks / 2 ? a.w2 : a.w;
-      if constexpr (TL) {
-        // unit sb / 2 (4608 bytes): page p's bytes 16 h .. in plane 2 (p % 2) + h, at 64 row + 32 (sb % 2) + 16 (p / 2);
-        // lane q reads page q / 2 (and 2 + q / 2), half q % 2: plane q
-        const u8 *u = m + (int64_t)(sb >> 1) * 4608;
-        c0[r & 1] = *reinterpret_cast<const uint4 *>(u + 32 * (sb & 1) + wr[r]);
-        c1[r & 1] = *reinterpret_cast<const uint4 *>(u + 32 * (sb & 1) + 16 + wr[r]);
-        hd[r & 1] = *reinterpret_cast<const uint4 *>(u + 16 * (sb & 1) + (wr[r] - hoff));
-      } else {
-        const u8 *b = m + (int64_t)sb * 144;
-        c0[r & 1] = *reinterpret_cast<const uint4 *>(b + 16 + (wr[r] + 16u * (u32)q));
-        c1[r & 1] = *reinterpret_cast<const uint4 *>(b + 80 + (wr[r] + 16u * (u32)q));
-        hd[r & 1] = *reinterpret_cast<const uint4 *>(b + wr[r]);
-      }
-    };
-    load_w(0);
-    u32 xb[NT][8][2];      // token codes of group g: two dwords
-    float sx[NT][2];       // xs da of the lane's token, groups q and q + 4
-    float *md = reinterpret_cast<float *>(own + kCode);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      uint4 v[4], m;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {   // 16 lanes a token: its 256 codes
-        const int tok = min(t0 + 16 * t + 4 * i + q, a.tokens - 1);
-        v[i] = *reinterpret_cast<const uint4 *>(a.codes + sb * 256 + ((u32)tok * K + 16u * (u32)c));
-      }
-      {                               // four lanes a token: its 8 pairs
-        const int tok = min(t0 + 16 * t + (lane >> 2), a.tokens - 1);
-        m = *reinterpret_cast<const uint4 *>(reinterpret_cast<const u8 *>(a.meta) + sb * 64 +
-                                             ((u32)tok * (K / 4u) + 16u * (u32)(lane & 3)));
-      }
-      // piece i of token k at i ^ k: the 16 tokens of a read lie in different banks
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<uint4 *>(own + (4 * i + q) * 256 + 16 * (c ^ (4 * i + q))) = v[i];
-      float *mt = md + 256 * t + 32 * (lane & 3) + (lane >> 2);   // groups 2 (lane % 4) and + 1, token lane / 4
-      const float d0 = u32_as_f32(m.x), d1 = u32_as_f32(m.z);
-      mt[0] = d0;
-      mt[16] = d1;
-      mt[128] = d0 * u32_as_f32(m.y);   // exact: 11 x 12 bits
-      mt[144] = d1 * u32_as_f32(m.w);
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  // ---- the waves' sums meet, in place of their own areas
+  __syncthreads();
+  hand(meet);
+  __syncthreads();
+  auto total = [&](const float *from, int o) __attribute__((always_inline)) {
+    if constexpr (ORDER == kItems) {   // the butterfly's steps 16 .. 1
+      float pv[4];
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
-        uint4 x = *reinterpret_cast<const uint4 *>(own + c * 256 + 16 * ((4 * p + q) ^ c));
-        page_swap(x.x, x.z);
-        page_swap(x.y, x.w);
-        xb[t][2 * p][0] = x.x; xb[t][2 * p][1] = x.y;
-        xb[t][2 * p + 1][0] = x.z; xb[t][2 * p + 1][1] = x.w;
+        auto w = [&](int k) { return from[(k * 4 + p) * 256 + o]; };
+        pv[p] = ((w(0) + w(4)) + (w(2) + w(6))) + ((w(1) + w(5)) + (w(3) + w(7)));
       }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) sx[t][j] = md[256 * t + 128 + 16 * (q + 4 * j) + c];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      return 0.f + ((pv[0] + pv[2]) + (pv[1] + pv[3]));
+    } else {                           // the slices in order
+      float s = 0.f;
+      for (int k = 0; k < a.nsb / per; ++k) s += from[k * 256 + o];
+      return s;
     }
-    // ---- the row blocks, the next one's loads in flight
-#pragma unroll
-    for (int r = 0; r < kRowBlocks; ++r) {
-      if (r + 1 < kRowBlocks) load_w(r + 1);
-      uint4 x = c0[r & 1], z = c1[r & 1];
-      const uint4 h = hd[r & 1];
-      page_swap(x.x, x.z);
-      page_swap(x.y, x.w);
-      page_swap(z.x, z.z);
-      page_swap(z.y, z.w);
-      const u32 pg[4][2] = {{x.x, x.y}, {x.z, x.w}, {z.x, z.y}, {z.z, z.w}};
-      // row c's scales of groups q and q + 4 (ggml get_scale_min_k4); the d sc go to the lanes that hold its sums
-      const u32 sh = 8u * (u32)q;
-      const u32 y0 = h.y >> sh, z0 = h.z >> sh, w0 = h.w >> sh;
-      const float d = f16_to_f32(h.x), dmin = f16_to_f32(h.x >> 16);
-      const float sc0 = d * (float)(y0 & 63u), sc1 = d * (float)((w0 & 15u) | ((y0 >> 2) & 48u));
-      const float mn0 = dmin * (float)(z0 & 63u) - 8.f * sc0, mn1 = dmin * (float)(((w0 >> 4) & 15u) | ((z0 >> 2) & 48u)) - 8.f * sc1;
-      float *sl = reinterpret_cast<float *>(own + kCode + kMeta);
-      sl[lane] = sc0 * 0.0625f;
-      sl[64 + lane] = sc1 * 0.0625f;
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      // a super-block's sum in two chains of four groups before it joins the wave's: short chains, and so rounding
-      // errors, as the matvec kernels' trees have them
-      f32x4 part[2][NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        part[0][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(-mn0, sx[t][0], zero, 0, 0, 0);
-        part[1][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(-mn1, sx[t][1], zero, 0, 0, 0);
-      }
-#pragma unroll
-      for (int g = 0; g < 8; ++g) {
-        const f32x4 s = *reinterpret_cast<const f32x4 *>(sl + 16 * g + 4 * q);   // rows 4 q .. 4 q + 3 of group g
-        const u32 e0 = pg[g >> 1][0], e1 = pg[g >> 1][1];
-        // 16 (q - 8) as int8: the nibble in the high half, its top bit flipped
-        const long wa = (g & 1) ? pack8((e0 & 0xF0F0F0F0u) ^ 0x80808080u, (e1 & 0xF0F0F0F0u) ^ 0x80808080u)
-                                : pack8(((e0 << 4) & 0xF0F0F0F0u) ^ 0x80808080u, ((e1 << 4) & 0xF0F0F0F0u) ^ 0x80808080u);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const float da = md[256 * t + 16 * g + c];
-          const i32x4 di = __builtin_amdgcn_mfma_i32_16x16x32_i8(wa, pack8(xb[t][g][0], xb[t][g][1]), i32x4{0, 0, 0, 0}, 0, 0, 0);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) part[g >> 2][t][i] = __builtin_fmaf((float)di[i], s[i] * da, part[g >> 2][t][i]);
-        }
-        if (g & 1) __builtin_amdgcn_sched_barrier(0);   // keeps the groups' LDS reads from piling up in registers
-      }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const f32x4 v = acc[r][t] + (part[0][t] + part[1][t]);
-        if constexpr (!kTwoSums) {
-          acc[r][t] = v;
-        } else {   // the two swap places after every super-block
-          acc[r][t] = alt[r][t];
-          alt[r][t] = v;
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    }
-  }
-
-  // ---- the waves' sums meet, two row blocks at a time (swiglu: a gate and its up block): [wave][block][token][row]
-  float *red = reinterpret_cast<float *>(smem);
-#pragma unroll
-  for (int rr = 0; rr < kRowBlocks / kPair; ++rr) {
-    __syncthreads();   // the waves' own areas (or the sums before) are done with
-#pragma unroll
-    for (int u = 0; u < kPair; ++u)
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        *reinterpret_cast<f32x4 *>(&red[((wave * kPair + u) * NT + t) * 256 + 16 * c + 4 * q]) =
-            SWIGLU ? acc[rr + kRowBlocks / 2 * u][t] : kTwoSums ? acc[kPair * rr + u][t] + alt[kPair * rr + u][t] : acc[kPair * rr + u][t];
+  };
+  const int o = tid & 255, tok = t0 + o / 16, rw = row0 + (o & 15);
+  const bool in = tok < a.tokens && rw < a.n;
+  if constexpr (SWIGLU) {   // threads 0 .. 255 the gate, the others the up total
+    const float s = total(tid < 256 ? meet_gate : meet, o);
     __syncthreads();
-    for (int o = tid; o < (SWIGLU ? 1 : kPair) * NT * 256; o += 64 * kWaves) {
-      auto total = [&](int at) {   // of the waves, as a tree
-        float e[kWaves];
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) e[w] = red[w * kPair * NT * 256 + at];
-        if constexpr (kWaves == 4) return (e[0] + e[1]) + (e[2] + e[3]);
-        else return ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
-      };
-      float v = total(o);
-      const int u = o / (NT * 256), tok = t0 + (o % (NT * 256)) / 16;
-      const int row = row0 + 16 * (SWIGLU ? rr : kPair * rr + u) + (o & 15);
-      if (tok < a.tokens && row < a.n) {
-        if constexpr (SWIGLU) v = act_fn(QMM_ACT_SILU, v, total(NT * 256 + o));
-        float *p = a.y + (int64_t)tok * a.n + row;
-        *p = a.accumulate ? *p + v : v;
-      }
+    if (tid >= 256) meet[o] = s;
+    __syncthreads();
+    if (tid < 256 && in) {
+      float *p = a.y + (int64_t)tok * a.n + rw;
+      const float y = act_fn(QMM_ACT_SILU, s, meet[o]);
+      *p = a.accumulate ? *p + y : y;
     }
+  } else if (tid < 256 && in) {
+    float *p = (blockIdx.y ? a.y2 : a.y) + (int64_t)tok * a.n + rw;
+    const float y = total(meet, o);
+    *p = a.accumulate ? *p + y : y;
   }
 }
 
-template <bool TL, bool SWIGLU, int NT, int R, int W>
-int launch(const MArgs &a, hipStream_t s) {
-  constexpr int kOut = 16 * (SWIGLU ? R / 2 : R);
-  const dim3 grid((unsigned)((a.n + kOut - 1) / kOut), (unsigned)((a.tokens + 16 * NT - 1) / (16 * NT)));
-  mv_q8_mfma_kernel<TL, SWIGLU, NT, R, W><<<grid, 64 * W, 0, s>>>(a);
+template <bool TL, int ORDER, bool LONG>
+int launch(int swiglu, MArgs a, hipStream_t s) {
+  a.tiles = (a.tokens + 15) / 16;
+  const dim3 grid((unsigned)(8 * ((a.n + 127) / 128) * a.tiles), a.y2 ? 2u : 1u);
+  if (swiglu) mv_q8_mfma_kernel<TL, true, ORDER, LONG><<<grid, 64 * kWaves, 0, s>>>(a);
+  else mv_q8_mfma_kernel<TL, false, ORDER, LONG><<<grid, 64 * kWaves, 0, s>>>(a);
   return launch_status();
 }
-// Eight waves a workgroup of 16 rows (swiglu: 16 of each matrix), so that 4096 rows fill the chip (with 64 rows a
-// workgroup 4096 x 4096 at 9 tokens took 15.2 us, with 16 7.9); swiglu past 16 tokens four waves, whose registers hold
-// both matrices' sums (eight would spill: 24 tokens 44.9 -> 26.5 us at 12288 x 4096; plain 20.6 us with eight waves, 28.4
-// with four at 4096 x 12288).
-template <bool TL, bool SWIGLU>
-int launch_nt(const MArgs &a, hipStream_t s) {
-  constexpr int R = SWIGLU ? 2 : 1;
-  return a.tokens <= 16 ? launch<TL, SWIGLU, 1, R, 8>(a, s) : launch<TL, SWIGLU, 2, R, SWIGLU ? 4 : 8>(a, s);
+
+// slices a wave of the tiled matvec kernel: K = 512 U NW, the least U <= 4 with NW <= 8 (qmm_mv_q4kt_q8); 0: none
+int tiled_slices(int64_t k) {
+  for (int u = 1; u <= 4; ++u)
+    if (k / 512 % u == 0 && k / 512 / u <= 8) return u;
+  return 0;
 }
 
 }  // namespace
 
 // Whether qmm_mv_q8_mfma takes a call (the int8 matvec entry points ask; their argument checks hold). Nine tokens and
-// more, and enough outputs for the grid: 1024 x 4096 at 24 tokens takes 9.4 us here, 9.0 in the matvec kernel; 4096 x 4096
-// 7.9 against 11.9 at nine tokens and 14.4 against 46.6 at 63; 12288 x 4096 gate / up 19.6 against 57.7 and 49 against 287
-// (Q4_K blocks; the tiled layout 17.5 against 36 and 45 against 160).
+// more, and enough outputs for the grid: 1024 x 4096 at 24 tokens takes 9.4 us here, 9.5 in the matvec kernel; 4096 x 4096
+// 8.1 against 14.0 at nine tokens and 16.2 against 71.8 at 63; 12288 x 4096 gate / up 21.9 against 52.7 and 65.8 against
+// 284 (Q4_K blocks; the tiled layout 21.7 against 34.8 and 62.0 against 153). Tiled rows of K < 2048 leave most waves
+// without a slice: 12288 gate / up at 24 tokens 20.1 against 17.5 at K = 512, 22.2 against 21.6 at 1024, 24.1 against 30.0
+// at 2048.
 // Shapes that the matvec kernels refuse (tiled: a K that does not split over their waves; too many rows) stay theirs.
 bool qmm_mv_q8_mfma_fits(int fmt, int64_t k, int64_t n, int64_t tokens) {
   if (fmt != QMM_Q4_K && fmt != QMM_Q4_KT) return false;
   if (k % 256 || tokens < 9 || n * tokens < 32768 || tokens > 65535 || n > 65535 * 8) return false;
   if (tokens * k >= (1ll << 31) || n * (k / 256 * 144) >= (1ll << 32)) return false;   // 32-bit byte offsets
   if (fmt == QMM_Q4_K) return true;
-  bool split = false;   // K = 512 U NW, U <= 4 slices a wave, NW <= 8 waves (qmm_mv_q4kt_q8)
-  for (int u = 1; u <= 4; ++u) split = split || (k / 512 % u == 0 && k / 512 / u <= 8);
-  return n % 16 == 0 && k % 512 == 0 && split;
+  return n % 16 == 0 && k % 512 == 0 && k >= 2048 && tiled_slices(k) > 0;
 }
 
-int qmm_mv_q8_mfma(int fmt, int swiglu, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *xq,
-                   const void *w, const void *w2, float *y, hipStream_t s) {
+// y2: a pair call (swiglu = 0). sliced: the call's one-token kernel is the K-sliced one (GGUF, K = 4096 or 8192).
+int qmm_mv_q8_mfma(int fmt, int swiglu, int sliced, int64_t k, int64_t n, int64_t tokens, int accumulate, const void *xq,
+                   const void *w, const void *w2, float *y, float *y2, hipStream_t s) {
   MArgs a{};
   a.n = (int)n; a.tokens = (int)tokens; a.nsb = (int)(k / 256);
   a.codes = static_cast<const u8 *>(xq);
   a.meta = reinterpret_cast<const float *>(a.codes + tokens * k);
   a.w = static_cast<const u8 *>(w); a.w2 = static_cast<const u8 *>(w2);
-  a.y = y; a.accumulate = accumulate;
-  if (fmt == QMM_Q4_KT) return swiglu ? launch_nt<true, true>(a, s) : launch_nt<true, false>(a, s);
-  return swiglu ? launch_nt<false, true>(a, s) : launch_nt<false, false>(a, s);
+  a.y = y; a.y2 = y2; a.accumulate = accumulate;
+  if (fmt == QMM_Q4_KT) {
+    a.chains = 2; a.units = tiled_slices(k);
+    return launch<true, kSlices, false>(swiglu, a, s);
+  }
+  if (sliced) {   // eight slices of 2 (K = 4096) or 4 super-blocks, a chain each
+    a.chains = (int)(k / 2048); a.units = 1;
+    return launch<false, kSlices, false>(swiglu, a, s);
+  }
+  return a.nsb > 2 * kWaves ? launch<false, kItems, true>(swiglu, a, s) : launch<false, kItems, false>(swiglu, a, s);
 }
