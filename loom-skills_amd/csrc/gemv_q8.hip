@@ -222,16 +222,17 @@ struct Q6K8 {
     x.da = live ? meta[2 * g] : 0.f;
     x.db = live ? meta[2 * g + 4] : 0.f;
   }
-  // unconditional (the callers clamp items and rows to real ones, whose x is zero or whose sums are not stored): loads
-  // in branches of their own would be waited for one by one
-  static __device__ __forceinline__ void load_w(const u8 *row, int item, bool, W &w) {
+  // unconditional (the callers clamp items and rows to real ones): loads in branches of their own would be waited for one
+  // by one. A lane past the row takes d = 0, as its x is: an infinite d would make its 0 a NaN
+  static __device__ __forceinline__ void load_w(const u8 *row, int item, bool live, W &w) {
     const u8 *b = row + (int64_t)(item >> 3) * 210;
     const int half = (item >> 2) & 1, i = item & 3;
     w.l = ld16u(b + 64 * half + 16 * i);
     w.h = ld16u(b + 128 + 32 * half + 16 * (i & 1));
     w.s0 = ld4u(b + 192 + 8 * half);
     w.s1 = ld4u(b + 196 + 8 * half);
-    w.d = *reinterpret_cast<const u16 *>(b + 208);
+    const u32 d = *reinterpret_cast<const u16 *>(b + 208);
+    w.d = live ? d : 0u;
   }
   static __device__ __forceinline__ float mac(const W &w, const X &x, int item, float acc) {
     const int g = (item >> 1) & 1, run = 2 * g + (item & 1);

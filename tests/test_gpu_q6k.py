@@ -202,3 +202,34 @@ def test_moe_prefill_q4_k_gate_up_q6_k_down(dev):
 
     want, _ = ref.moe(bf16_values(xb), eids, ewts, gate_up, down, x_round=ref.f16_rows, act_round=ref.f16_rows)
     assert_close_rel_l2(host(y), want, 1e-3, "q4_k/q6_k moe prefill")
+
+
+def _inf_rows(rng, n, k, super_block):
+    """Q6_K rows whose given super-block has an infinite d (negative in odd rows), codes 31 and scales 5."""
+    from qmm import synth
+    w = synth.q6_k_weights(rng, n, k).reshape(n, k // 256, 210)
+    w[:, super_block, :192] = 255
+    w[:, super_block, 192:208] = 5
+    w[:, super_block, 208] = 0
+    w[:, super_block, 209] = np.where(np.arange(n) % 2, 0xFC, 0x7C)
+    return w.reshape(-1), np.where(np.arange(n) % 2, -np.inf, np.inf).astype(np.float32)
+
+
+@pytest.mark.parametrize("n,k,m", [(50, 768, 1), (50, 2560, 1), (50, 2560, 3), (33000, 2560, 2)])
+def test_q6_k_q8_infinite_scale(dev, n, k, m):
+    """An infinite d in a row's last super-block gives that infinity, also where the row's item count leaves lanes
+    without an item (K = 768: 24 items, 2560: 80), a row a wave and four rows a wave; and in the expert matvecs."""
+    import torch
+    rng = np.random.default_rng(n + k + m)
+    ops = _ops()
+    w, want = _inf_rows(rng, n, k, -1)
+    wt, xt = dev_u8(w, dev), dev_f32(np.ones((m, k), np.float32), dev)
+    y = host(ops.mv_q8("q6_k", wt, xt, n, k))
+    np.testing.assert_array_equal(y, np.broadcast_to(want, (m, n)))
+    a, b = ops.mv_pair_q8("q6_k", wt, wt, xt, n, k)
+    np.testing.assert_array_equal(host(a), y)
+    np.testing.assert_array_equal(host(b), y)
+    if n < 100:
+        ids = torch.zeros((m, 1), dtype=torch.int32, device=dev)
+        e = host(ops.moe_expert_mv_q8("q6_k", "dn", ids, xt, wt, n, k, 1, 1))
+        np.testing.assert_array_equal(e, y)
