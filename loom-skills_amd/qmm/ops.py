@@ -137,11 +137,11 @@ def quant_q8(x, xq=None):
 def mv_q8(fmt, w, x, n, k, tokens=None, y=None, accumulate=False, ws=None):
     """The int8-activation decode matvec (g_mv_{fmt}_k{K}[_t{TG}]_q8, S/gen_llm.py:1288-1301): x is the planar Q8_1
     buffer of `tokens` rows (uint8, from quant_q8), or f32 / bf16 rows [tokens, k], which the Q4_K K = 4096 / 8192
-    and (up to two tokens) tiled-layout q4_kt / q4_0t kernels quantize themselves and any other call quantizes through
-    quant_q8 first (identical results). mxfp4s (the reference's opt-in MXFP4S_Q8): w the nibble plane, ws the E8M0
-    plane."""
+    kernel (up to eight tokens, and past them below 32768 outputs) and (up to two tokens) tiled-layout q4_kt / q4_0t
+    kernels quantize themselves and any other call quantizes through quant_q8 first (identical results). mxfp4s (the
+    reference's opt-in MXFP4S_Q8): w the nibble plane, ws the E8M0 plane."""
     _dev(w, ws, x, y)
-    x, xd, tokens = _q8_input(fmt, x, k, tokens, staged_tokens=2)
+    x, xd, tokens = _q8_input(fmt, x, n, k, tokens, staged_tokens=2)
     y = _out(y, (tokens, n), torch.float32, w.device, accumulate)
     if fmt == "mxfp4s":
         _split_q8(0, k, n, tokens, accumulate, x, xd, w, ws, None, None, y, None)
@@ -161,10 +161,11 @@ def _split_q8(mode, k, n, tokens, accumulate, x, xd, w, ws, w2, ws2, y, y2):
 TILED_Q8 = ("q4_kt", "q4_0t")   # the tiled layouts of the int8 matvec, which quantize f32 / bf16 rows themselves
 
 
-def _q8_input(fmt, x, k, tokens, staged_tokens):
-    """(x, its dtype code, tokens) for an int8 matvec: a planar Q8_1 buffer as it is (uint8, `tokens` rows), or f32 /
-    bf16 rows, which the Q4_K K = 4096 / 8192 and (up to `staged_tokens` tokens) tiled-layout kernels quantize
-    themselves and every other call quantizes through quant_q8 first (identical results)."""
+def _q8_input(fmt, x, n, k, tokens, staged_tokens):
+    """(x, its dtype code, tokens) for an int8 matvec of n rows: a planar Q8_1 buffer as it is (uint8, `tokens` rows), or
+    f32 / bf16 rows, which the Q4_K K = 4096 / 8192 kernel (where qmm_mv_q8 does not take the planar buffer to the int8
+    MFMA) and (up to `staged_tokens` tokens) the tiled-layout kernels quantize themselves and every other call quantizes
+    through quant_q8 first (identical results)."""
     if x.dtype == torch.uint8:
         if tokens is None:
             raise ValueError("a planar Q8_1 buffer needs its token count")
@@ -175,9 +176,12 @@ def _q8_input(fmt, x, k, tokens, staged_tokens):
     tokens = x.shape[0]
     _cols(x, k)
     # the kernels that quantize f32 / bf16 rows themselves do so in every workgroup; from three tokens on a separate
-    # quant_q8 pass is cheaper for the tiled layout (same bits either way), and from nine on the int8 MFMA kernel takes
-    # the planar buffer
-    if (fmt == "q4_k" and k in (4096, 8192) and staged_tokens >= 2 and tokens <= 8) or (fmt in TILED_Q8 and tokens <= staged_tokens):
+    # quant_q8 pass is cheaper for the tiled layout (same bits either way). The int8 MFMA kernel takes planar buffers of
+    # nine tokens and more with 32768 outputs (qmm_mv_q8_mfma_fits); with fewer the second launch only costs: Q4_K
+    # 1024 x 4096 at nine tokens 6.8 us in one launch, 7.3 in two, 512 x 4096 5.3 and 6.5
+    mfma = 9 <= tokens <= 65535 and n * tokens >= 32768
+    stages = fmt == "q4_k" and k in (4096, 8192) and staged_tokens >= 2 and not mfma
+    if stages or (fmt in TILED_Q8 and tokens <= staged_tokens):
         return x, _dt(x), tokens
     return quant_q8(x), DTYPE["q8"], tokens
 
@@ -187,7 +191,7 @@ def mv_swiglu_q8(fmt, w, w2, x, n, k, tokens=None, y=None, accumulate=False, ws=
     [n, k]; x a planar Q8_1 buffer (with tokens) or f32 / bf16 rows (quantized as quant_q8 does). fmt q4_kt / q4_0t
     (tiled layouts), GGUF q4_k / q4_0 / q6_k, or mxfp4s with ws / ws2 the scale planes. Returns y f32 [tokens, n]."""
     _dev(w, w2, ws, ws2, x, y)
-    x, xd, tokens = _q8_input(fmt, x, k, tokens, staged_tokens=2 if fmt in TILED_Q8 else 0)
+    x, xd, tokens = _q8_input(fmt, x, n, k, tokens, staged_tokens=2 if fmt in TILED_Q8 else 0)
     y = _out(y, (tokens, n), torch.float32, w.device, accumulate)
     if fmt == "mxfp4s":
         _split_q8(1, k, n, tokens, accumulate, x, xd, w, ws, w2, ws2, y, None)
@@ -202,7 +206,7 @@ def mv_pair_q8(fmt, w, w2, x, n, k, tokens=None, y=None, y2=None, accumulate=Fal
     each equal bit for bit to the one-matrix kernel's of the same layout (mxfp4s: ws / ws2 the scale planes).
     Returns (y, y2) f32 [tokens, n]."""
     _dev(w, w2, ws, ws2, x, y, y2)
-    x, xd, tokens = _q8_input(fmt, x, k, tokens, staged_tokens=2 if fmt in TILED_Q8 else 0)
+    x, xd, tokens = _q8_input(fmt, x, n, k, tokens, staged_tokens=2 if fmt in TILED_Q8 else 0)
     y = _out(y, (tokens, n), torch.float32, w.device, accumulate)
     y2 = _out(y2, (tokens, n), torch.float32, w.device, accumulate)
     if fmt == "mxfp4s":
