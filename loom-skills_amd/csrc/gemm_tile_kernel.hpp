@@ -32,7 +32,6 @@
 // 64 jh + 32 h + 16 gl + 8 s2 .. . The activation fragment is read from LDS at the same K.
 #pragma once
 
-
 #include <type_traits>
 
 #include "common.hpp"
@@ -55,7 +54,7 @@ __device__ __forceinline__ void lds_load16(u32x4 rsrc, u32 voff, u32 soff, u32 l
   asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                :
                : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds)
-               : "memory");
+               : "m0", "memory");
 }
 __device__ __forceinline__ void wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
