@@ -439,13 +439,15 @@ int tile_gemm(int fmt, int kind, int shape, const TileArgs &a, hipStream_t s) {
 }
 
 // The workgroup shape of a dense GEMM: the least ceil(tiles / 256 CUs) x (time of a CU's tile). Times in units of us at
-// K = 4096 (Q4_K; the ratios hold for the other formats and K within some 10 %), measured with a full chip: a 128 x 256
-// tile 64 (two workgroups a CU) or, K in two parts, 70 (58 where one round does), a 64 x 256 tile 41 (46), a 64 x 128
-// tile with K in four parts 30; the Q4_K store / acc kernel of gemm_dense.hip 26. So 2048 x 4096 outputs take the
-// two-part 128-row tiles (K = 12288: 194 us; 210 one part, 239 and 296 on 64 rows, 270 gemm_dense.hip), 2048 x 12288
-// one part (204; 222, 243, 359, 339), 333 x 12288 gate / up the 64 x 256 tiles (109; 113, 121, 140).
+// K = 4096 on Q4_K, measured with a full chip: a 128 x 256 tile 64 (two workgroups a CU) or, K in two parts, 70 (58 where
+// one round does), a 64 x 256 tile 41 (46), a 64 x 128 tile with K in four parts 30; the Q4_K store / acc kernel of
+// gemm_dense.hip 26. So 2048 x 4096 outputs take the two-part 128-row tiles (Q6_K, K = 12288: 194 us; 210 one part, 239
+// and 296 on 64 rows), 2048 x 12288 one part (204; 222, 243, 359), 333 x 12288 gate / up the 64 x 256 tiles (109; 113,
+// 121, 140). Two rounds of gemm_dense.hip overlap, the more the longer they are: 1024 x 4096 outputs of Q4_K take it 39, 66
+// and 151 us at K = 1024, 4096 and 12288, the 64 x 256 tiles 29, 71 and 190. A row's K-parts, and so the order of its
+// sums, follow from the shape: its last bits depend on the number of rows it comes with.
 constexpr int kDenseKernel = -1;
-int tile_shape(bool two, bool q4k, int64_t m, int64_t n) {
+int tile_shape(bool two, bool q4k, int64_t m, int64_t n, int64_t k) {
   const int64_t cols = two ? 2 * n : n, m64 = (m + 63) / 64, m128 = (m + 127) / 128;
   const int64_t n128 = (cols + 127) / 128, n256 = (cols + 255) / 256;
   auto rounds = [](int64_t tiles) { return (tiles + 255) / 256; };
@@ -458,7 +460,7 @@ int tile_shape(bool two, bool q4k, int64_t m, int64_t n) {
   offer(kT128x4x2, r0 == 1 ? 58 : 70 * r0);
   offer(kT64x4x1, r2 == 1 ? 46 : 41 * r2);
   offer(kT64x2x4, 30 * r3);
-  if (q4k && !two) offer(kDenseKernel, 26 * r3);
+  if (q4k && !two) offer(kDenseKernel, r3 == 2 && k >= 3072 ? 44 : 26 * r3);
   return best;
 }
 int fmt_align(int fmt) { return fmt == QMM_Q4_K || fmt == QMM_Q4_KT ? 16 : fmt == QMM_Q6_K ? 4 : 2; }
@@ -503,7 +505,7 @@ extern "C" int qmm_gemm(int fmt, int mode, int64_t rows, int64_t k, int64_t n, c
     a.tiles_total = a.tiles_m * (int)((n + 63) / 64);   // 64 output columns a workgroup: wave pairs take gate and up
     return bf ? launch_mixed<kSwiglu, true>(fmt, fu, a, s) : launch_mixed<kSwiglu, false>(fmt, fu, a, s);
   }
-  const int shape = tile_shape(mode == QMM_GEMM_SWIGLU, fmt == QMM_Q4_K || tiled, rows, n);
+  const int shape = tile_shape(mode == QMM_GEMM_SWIGLU, fmt == QMM_Q4_K || tiled, rows, n, k);
   if (shape == kDenseKernel) return qmm_gemm_q4k_dense(acc, tiled, rows, k, n, x, scales, w, y, bf, s);
   TileArgs t{};
   t.M = (int)rows; t.N = (int)n; t.K = (int)k;
