@@ -66,7 +66,7 @@ def _call(fmt, mode, xt, w, N, K, y0=None):
     ("q4_k", 9, 3700, 256), ("q4_k", 33, 1005, 1280), ("q4_k", 16, 2056, 2560),     # up to one super-block an item lane
     ("q4_k", 24, 1400, 4352), ("q4_k", 11, 3001, 12288),                             # several
     ("q4_k", 17, 2050, 4096), ("q4_k", 63, 528, 4096), ("q4_k", 12, 2800, 8192),     # K slices (swiglu: items)
-    ("q4_kt", 9, 3712, 512), ("q4_kt", 20, 1648, 2560), ("q4_kt", 33, 1008, 4096),   # one tiled slice a wave
+    ("q4_kt", 9, 3712, 1024), ("q4_kt", 20, 1648, 2560), ("q4_kt", 33, 1008, 4096),   # one tiled slice a wave
     ("q4_kt", 16, 2048, 5120), ("q4_kt", 40, 832, 12288)])                           # two, three
 @pytest.mark.parametrize("mode", ["store", "acc", "swiglu", "pair"])
 def test_multi_token_equals_one_token(dev, fmt, mode, M, N, K):
