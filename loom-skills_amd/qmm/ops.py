@@ -179,9 +179,10 @@ def _q8_input(fmt, x, n, k, tokens, staged_tokens):
     # quant_q8 pass is cheaper for the tiled layout (same bits either way). The int8 MFMA kernel takes planar buffers of
     # nine tokens and more with 32768 outputs (qmm_mv_q8_mfma_fits); with fewer the second launch only costs: Q4_K
     # 1024 x 4096 at nine tokens 6.8 us in one launch, 7.3 in two, 512 x 4096 5.3 and 6.5
-    mfma = 9 <= tokens <= 65535 and n * tokens >= 32768
-    stages = fmt == "q4_k" and k in (4096, 8192) and staged_tokens >= 2 and not mfma
-    if stages or (fmt in TILED_Q8 and tokens <= staged_tokens):
+    if fmt == "q4_k":
+        if k in (4096, 8192) and staged_tokens >= 2 and (tokens <= 8 or tokens > 65535 or n * tokens < 32768):
+            return x, _dt(x), tokens
+    elif fmt in TILED_Q8 and tokens <= staged_tokens:
         return x, _dt(x), tokens
     return quant_q8(x), DTYPE["q8"], tokens
 
