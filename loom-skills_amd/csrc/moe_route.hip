@@ -920,7 +920,7 @@ static int router(int64_t tokens, int64_t H, int E, const void *x, int x_dtype, 
   };
   auto shape = [&](auto xc, auto wc) {
     using std::integral_constant;
-    // 8 x 8 from where its waves fill the chip's 1024 SIMDs (E = 128: 512 tokens), 4 x 4 from a quarter of that
+    // 8 x 8 from where its waves fill the chip's 1024 SIMDs (E = 128: 512 tokens), 4 x 4 from half of them (64 tokens)
     const int64_t outs = tokens * E;
     if (E >= 8 && outs >= 65536) go(xc, wc, integral_constant<int, 8>{}, integral_constant<int, 8>{});
     else if (E >= 4 && outs >= 8192) go(xc, wc, integral_constant<int, 4>{}, integral_constant<int, 4>{});

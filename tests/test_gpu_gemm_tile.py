@@ -1,6 +1,6 @@
 """GPU parity of the tile GEMM's workgroup shapes (qmm_gemm picks one by the tile count): every format and mode at sizes
-that take each shape, with partial row and column tiles, K-parts of unequal and zero length, and 64-row runs of padding
-rows inside a 128-row tile. Oracle: the float64 product of the f16 operand and the exactly dequantized weights, rel-L2
+that take each shape (Q4_K store / acc: the first four the kernel of gemm_dense.hip), with partial row and column tiles,
+K-parts of unequal and zero length, and 64-row runs of padding rows inside a 128-row tile. Oracle: the float64 product of the f16 operand and the exactly dequantized weights, rel-L2
 1e-3 (f16 weights round at 2^-11: 2.8e-4 rms, 4e-4 for the product of two such sums)."""
 import numpy as np
 import pytest
@@ -15,7 +15,8 @@ SIZES = [(64, 128, 256),       # 64 x 128 tiles, four K-parts of which two are e
          (77, 145, 768),       # the same, parts of one and two steps
          (200, 129, 1280),     # a last row tile of eight rows (one 32-row block)
          (300, 4097, 256),     # 64 x 256 tiles as gate / up
-         (1100, 4001, 512),    # 128 x 256 tiles, two K-parts
+         (300, 8190, 256),     # 64 x 256 tiles; as gate / up 128 x 256 tiles, two K-parts of one step each
+         (1100, 4001, 512),    # 128 x 256 tiles, two K-parts; as gate / up 64 x 256
          (4090, 3327, 256)]    # 128 x 256 tiles, one K-part
 
 
