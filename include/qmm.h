@@ -141,9 +141,12 @@ int qmm_mv_pair_q8(int fmt, int64_t k, int64_t n, int64_t tokens, int accumulate
  *   swiglu: Y = silu((X W^T) inv) * ((X W2^T) inv)
  * x: f16 [rows, k] (x_dtype QMM_F16), the reference's row-scaled x16 from qmm_row_scale_f16; scales: f32 [rows, 2]
  * with inv = scales[row, 1] (the reference's (2^-e, 2^e) pairs), or NULL for inv = 1; y: [rows, n] of y_dtype
- * (QMM_F32 as the reference, or QMM_BF16, rounded to nearest even). fp32 accumulation. K % 256 == 0. Weights are
+ * (QMM_F32 as the reference, or QMM_BF16, rounded to nearest even). fp32 accumulation; the parts K is summed in follow
+ * from (rows, n, k), so a row's last bits can depend on the number of rows it comes with. K % 256 == 0. Weights are
  * dequantized to f16 as the reference stages them: Q4_K fma_f16(f16(q), f16(d sc), f16(-dmin m)); Q6_K (fmt
- * QMM_Q6_K, S/gen_gemm.py:369-444) fma_f16(f16(q), f16(d sc), f16(-32 d sc)) with q the unsigned 6-bit code; Q4_0
+ * QMM_Q6_K, S/gen_gemm.py:369-444) f16(f16(d sc) (q - 32)) with q the unsigned 6-bit code, which is the reference's
+ * fma_f16(f16(q), f16(d sc), f16(-32 d sc)) where f16(d sc) is normal and -32 d sc finite in f16, and nearer to
+ * d sc (q - 32) elsewhere (a QMM_GATE_UP pair's Q6_K matrix takes the reference's form everywhere); Q4_0
  * (fmt QMM_Q4_0, the reference's native Q4_0 staging S/moe_q4_0.py:11-38, S/gen_gemm.py:40-45) f16(q - 8) * d with
  * one f16 rounding, i.e. f16(d (q - 8)) for every finite d. MXFP4 weights go through qmm_gemm_mxfp4.
  * fmt QMM_Q4_KT: Q4_K in the tiled layout of qmm_tile_q4k (the int8 decode GEMV's; n % 16 == 0, K % 512 == 0), the

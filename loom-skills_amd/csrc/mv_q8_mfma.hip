@@ -18,8 +18,8 @@
 // The matvec kernels read every weight once per two tokens (GGUF) or eight (tiled) and spend a v_dot4 per four products.
 // Here a weight is read once per 16 tokens and 16 x 16 products of a group take one v_mfma_i32_16x16x32_i8 a wave: what is
 // left is the fixup of each group's 256 sums (convert, two fma; kItems half a multiply and half an add more: 12 - 14 vector
-// instructions of a wave's 30 a group), which bounds it: 24 tokens through 2 x 12288 x 4096 keep the vector pipes busy 76 %
-// of the time a CU holds a wave, the LDS 46 %. That call: 112 us in the matvec kernel, 30.4 here, with the quantizer's
+// instructions of a wave's 30 a group), which bounds it: 24 tokens through 2 x 12288 x 4096 keep the vector pipes busy 80 %
+// of the time a CU holds a wave, the address unit 73 %, the LDS 48 %. That call: 112 us in the matvec kernel, 30.4 here, with the quantizer's
 // launch (8 us of weights).
 //
 // A workgroup: 16 weight rows (swiglu: of each matrix) x 16 tokens, eight waves. A wave takes whole super-blocks of all rows

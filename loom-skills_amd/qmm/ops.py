@@ -203,8 +203,9 @@ def mv_swiglu_q8(fmt, w, w2, x, n, k, tokens=None, y=None, accumulate=False, ws=
 
 
 def mv_pair_q8(fmt, w, w2, x, n, k, tokens=None, y=None, y2=None, accumulate=False, ws=None, ws2=None):
-    """Two int8 matvecs of one input in one launch (g_mv_{fmt}_k{K}_pair[_t{TG}]_q8): y (+)= x W^T, y2 (+)= x W2^T,
-    each equal bit for bit to the one-matrix kernel's of the same layout (mxfp4s: ws / ws2 the scale planes).
+    """Two int8 matvecs of one input in one launch, past the quantizer's where rows need one
+    (g_mv_{fmt}_k{K}_pair[_t{TG}]_q8): y (+)= x W^T, y2 (+)= x W2^T, each equal bit for bit to
+    the one-matrix kernel's of the same layout (mxfp4s: ws / ws2 the scale planes).
     Returns (y, y2) f32 [tokens, n]."""
     _dev(w, w2, ws, ws2, x, y, y2)
     x, xd, tokens = _q8_input(fmt, x, n, k, tokens, staged_tokens=2 if fmt in TILED_Q8 else 0)
